@@ -1,0 +1,1176 @@
+// Device code shared by the stage kernels: fluxes, ghost states, gradients and limiters,
+// reconstruction, the cell update and the RMS leaf sums.  Included by every kernel file, so
+// each of them runs the same arithmetic.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <cmath>
+#include <cstdint>
+#include <type_traits>
+
+#include "dev.hpp"
+
+namespace ebb {
+
+#define DEV __device__ __forceinline__
+constexpr double G_ = 1.4;
+constexpr int BLK = 256;
+static_assert(uint32_t(BLK) == FACE_TILE_LANES, "face tile padding assumes one lane per workgroup thread");
+constexpr int FORCE_LDS = 1024;   // force faces staged per pass by a gradient kernel's force workgroup
+
+enum { BT_FULL = 0, BT_CONSTP, BT_INVWALL, BT_VISCWALL, BT_SYM, BT_TPIN, BT_DIRICHLET };
+
+// workgroup b runs on XCD b % 8; hand each XCD a contiguous slice of the cells
+DEV uint32_t xcdBlock(uint32_t b, uint32_t nb)
+{
+    const uint32_t nx = 8, per = nb / nx, rem = nb % nx, x = b % nx, k = b / nx;
+    return x * per + (x < rem ? x : rem) + k;
+}
+
+// The same slices, each walked last to first (the k-th workgroup of XCD x takes the k-th
+// item from its slice's end; k < the slice's length for every b < nb)
+DEV uint32_t xcdBlockBack(uint32_t b, uint32_t nb)
+{
+    const uint32_t nx = 8, per = nb / nx, rem = nb % nx, x = b % nx, k = b / nx;
+    const uint32_t len = per + (x < rem ? 1u : 0u);
+    return x * per + (x < rem ? x : rem) + (len - 1 - k);
+}
+
+// The face, reconstruction and limiter arithmetic below is written once for the
+// real type R it computes in: double on the FP64 path, float on the mixed path
+// (extensions.precision = "mixed").  Every literal is converted to R, so the double
+// instantiation performs exactly the operations of the FP64 path and the float one
+// never promotes to double.
+template <typename R>
+DEV R pressure(const R q[4])
+{
+    const R a = q[1] / q[0], b = q[2] / q[0];
+    return R(G_ - 1) * (q[3] - R(0.5) * q[0] * (a * a + b * b));
+}
+
+template <typename R>
+DEV R dmax(R a, R b) { return a < b ? b : a; }
+
+template <typename R>
+DEV R harten(R lam, R eps)
+{
+    if (lam < eps) lam = (eps * eps + lam * lam) / (R(2.0) * eps);
+    return lam;
+}
+
+// flux.d:19-24
+template <typename R>
+DEV void convective(R p, R u, R v, R rho, R e, R n0, R n1, R out[4])
+{
+    out[0] = (rho * u) * n0 + (rho * v) * n1;
+    out[1] = (p + rho * (u * u)) * n0 + (rho * u * v) * n1;
+    out[2] = (rho * u * v) * n0 + (p + rho * (v * v)) * n1;
+    out[3] = (u * (p + e)) * n0 + (v * (p + e)) * n1;
+}
+
+// flux.d:224-303
+template <typename R>
+DEV void roeFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
+{
+    const R gm1 = R(G_ - 1), half = R(0.5);
+    const R rhoL = qL[0], uL = qL[1] / rhoL, vL = qL[2] / rhoL;
+    const R rvL0 = rhoL * uL, rvL1 = rhoL * vL;
+    const R pL = (gm1 * (qL[3] - half * rhoL * (uL * uL + vL * vL)));
+    const R hL = (qL[3] + pL) / rhoL;
+    const R rhoR = qR[0], uR = qR[1] / rhoR, vR = qR[2] / rhoR;
+    const R rvR0 = rhoR * uR, rvR1 = rhoR * vR;
+    const R pR = (gm1 * (qR[3] - half * rhoR * (uR * uR + vR * vR)));
+    const R hR = (qR[3] + pR) / rhoR;
+    const R di = sqrt(rhoR / rhoL);
+    const R d1 = R(1.0) / (R(1.0) + di);
+    const R vel0 = (di * uR + uL) * d1, vel1 = (di * vR + vL) * d1;
+    const R u = vel0 * n0 + vel1 * n1;
+    const R h = (di * hR + hL) * d1;
+    const R a = sqrt(R(G_ - 1.0) * (h - half * (vel0 * vel0 + vel1 * vel1)));
+    const R dRhoV0 = rvR0 - rvL0, dRhoV1 = rvR1 - rvL1;
+    const R dRho = rhoR - rhoL, dRhoE = qR[3] - qL[3];
+    const R eps = R(0.01) * a;
+    const R lam1 = harten<R>(fabs(u + a), eps);
+    const R lam2 = harten<R>(fabs(u - a), eps);
+    const R lam3 = harten<R>(fabs(u), eps);
+    const R lam4 = harten<R>(fabs(u), eps);
+    sMax = dmax<R>(dmax<R>(dmax<R>(fabs(lam1), fabs(lam2)), fabs(lam3)), fabs(lam4));
+    const R s1 = half * (lam1 + lam2), s2 = half * (lam1 - lam2);
+    const R qq = sqrt(vel0 * vel0 + vel1 * vel1);
+    const R G1 = gm1 * (((qq * qq) / R(2.0)) * dRho - (vel0 * dRhoV0 + vel1 * dRhoV1) + dRhoE);
+    const R G2 = -u * dRho + (dRhoV0 * n0 + dRhoV1 * n1);
+    const R C1 = (G1 / (a * a)) * (s1 - lam3) + G2 / a * s2;
+    const R C2 = (G1 / a) * s2 + (s1 - lam3) * G2;
+    R fL[4], fR[4];
+    convective<R>(pL, uL, vL, rhoL, qL[3], n0, n1, fL);
+    convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
+    const R d[4] = {lam3 * dRho + C1, lam3 * dRhoV0 + C1 * vel0 + C2 * n0,
+                    lam3 * dRhoV1 + C1 * vel1 + C2 * n1, lam3 * dRhoE + C1 * h + C2 * u};
+#pragma unroll
+    for (int k = 0; k < 4; k++) out[k] = half * (fL[k] + fR[k]) - half * d[k];
+}
+
+// flux.d:66-141 (Roe-type averages, C1 = C2 = 0: central flux + sMax jump)
+template <typename R>
+DEV void rusanovFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
+{
+    const R gm1 = R(G_ - 1), half = R(0.5);
+    const R rhoL = qL[0], uL = qL[1] / rhoL, vL = qL[2] / rhoL;
+    const R rvL0 = rhoL * uL, rvL1 = rhoL * vL;
+    const R pL = (gm1 * (qL[3] - half * rhoL * (uL * uL + vL * vL)));
+    const R hL = (qL[3] + pL) / rhoL;
+    const R rhoR = qR[0], uR = qR[1] / rhoR, vR = qR[2] / rhoR;
+    const R rvR0 = rhoR * uR, rvR1 = rhoR * vR;
+    const R pR = (gm1 * (qR[3] - half * rhoR * (uR * uR + vR * vR)));
+    const R hR = (qR[3] + pR) / rhoR;
+    const R rho = sqrt(rhoL * rhoR);
+    const R sL = sqrt(rhoL), sR = sqrt(rhoR);
+    const R vel0 = (sL * uL + sR * uR) / (sL + sR);
+    const R vel1 = (sL * vL + sR * vR) / (sL + sR);
+    const R u = vel0 * n0 + vel1 * n1;
+    const R p = (sL * pL + sR * pR) / (sL + sR);
+    const R h = (sL * hL + sR * hR) / (sL + sR);
+    const R a = sqrt(R(G_) * (p / rho));
+    const R dRhoV0 = rvR0 - rvL0, dRhoV1 = rvR1 - rvL1;
+    const R dRho = rhoR - rhoL, dRhoE = qR[3] - qL[3];
+    const R eps = R(0.01) * a;
+    const R lam1 = harten<R>(fabs(u + a), eps);
+    const R lam2 = harten<R>(fabs(u - a), eps);
+    const R lam3 = harten<R>(fabs(u), eps);
+    const R lam4 = harten<R>(fabs(u), eps);
+    const R sm = dmax<R>(dmax<R>(dmax<R>(fabs(lam1), fabs(lam2)), fabs(lam3)), fabs(lam4));
+    sMax = sm;
+    const R s1 = half * (sm + sm), s2 = half * (sm - sm);
+    const R qq = sqrt(vel0 * vel0 + vel1 * vel1);
+    const R G1 = gm1 * ((qq * qq / R(2)) * dRho - (vel0 * dRhoV0 + vel1 * dRhoV1) + dRhoE);
+    const R G2 = -u * dRho + (dRhoV0 * n0 + dRhoV1 * n1);
+    const R C1 = (G1 / (a * a)) * (s1 - sm) + G2 / a * s2;
+    const R C2 = (G1 / a) * s2 + (s1 - sm) * G2;
+    R fL[4], fR[4];
+    convective<R>(pL, uL, vL, rhoL, qL[3], n0, n1, fL);
+    convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
+    const R d[4] = {sm * dRho + C1, sm * (dRhoV0) + C1 * vel0 + C2 * n0,
+                    sm * (dRhoV1) + C1 * vel1 + C2 * n1, sm * dRhoE + C1 * h + C2 * u};
+#pragma unroll
+    for (int k = 0; k < 4; k++) out[k] = half * (fL[k] + fR[k]) - half * d[k];
+}
+
+template <int FLUX, typename R>
+DEV void numFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
+{
+    if (FLUX == 1) roeFlux<R>(qL, qR, n0, n1, out, sMax);
+    else rusanovFlux<R>(qL, qR, n0, n1, out, sMax);
+}
+
+// flux.d:28-64.  The four 4x4 matrices are applied entry by entry in column
+// order; their structural zeros only ever add a signed zero, so they are skipped.
+// Pr and mu are physical parameters (FP64), converted to R.
+template <typename R>
+DEV void viscousFlux(double Prd, double mud, const R q[4], const R dq[8], R n0, R n1, R out[4])
+{
+    const R rho = q[0], u = q[1] / q[0], v = q[2] / q[0], E = q[3] / q[0];
+    const R gp = R(G_) / R(Prd);
+    const R s = R(mud) / rho;
+    const R one = R(1.0);
+    const R c43 = R(4.0 / 3.0), c23 = R(2.0 / 3.0), cm43 = R(-4.0 / 3.0), cm23 = R(-2.0 / 3.0), c231 = R(2.0 / 3.0 - 1.0);
+    const R t0 = (cm43 + gp) * (u * u) + (-one + gp) * (v * v) - gp * E;
+    const R t1 = (-one + gp) * (u * u) + (cm43 + gp) * (v * v) - gp * E;
+    const R x0 = dq[0], x1 = dq[2], x2 = dq[4], x3 = dq[6];
+    const R y0 = dq[1], y1 = dq[3], y2 = dq[5], y3 = dq[7];
+    const R uv = c231 * u * v;
+    const R G01 = ((s * (cm43 * u)) * x0 + (s * c43) * x1) + ((s * (c23 * v)) * y0 + (s * cm23) * y2);
+    const R G02 = ((s * -v) * x0 + (s * one) * x2) + ((s * -u) * y0 + (s * one) * y1);
+    const R G03 = ((s * t0) * x0 + (s * ((c43 - gp) * u)) * x1 + (s * ((one - gp) * v)) * x2 + (s * gp) * x3)
+                + ((s * uv) * y0 + (s * v) * y1 + (s * (cm23 * u)) * y2);
+    const R G11 = ((s * -v) * x0 + (s * one) * x2) + ((s * -u) * y0 + (s * one) * y1);
+    const R G12 = ((s * (c23 * u)) * x0 + (s * cm23) * x2) + ((s * (cm43 * v)) * y0 + (s * c43) * y2);
+    const R G13 = ((s * uv) * x0 + (s * (cm23 * v)) * x1 + (s * u) * x2)
+                + ((s * t1) * y0 + (s * ((one - gp) * u)) * y1 + (s * ((c43 - gp) * v)) * y2 + (s * gp) * y3);
+    out[0] = R(0.0);
+    out[1] = G01 * n0 + G11 * n1;
+    out[2] = G02 * n0 + G12 * n1;
+    out[3] = G03 * n0 + G13 * n1;
+}
+
+DEV void ld4(const double4* p, uint32_t i, double o[4])
+{
+    const double4 t = p[i];
+    o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
+}
+DEV void st4(double4* p, uint32_t i, const double o[4]) { p[i] = make_double4(o[0], o[1], o[2], o[3]); }
+// gradients and limiters are read once, by the next kernel: stored non-temporally so
+// they do not displace the neighbour data that kernel's gathers reuse from L2
+typedef double ntd2 __attribute__((ext_vector_type(2)));
+typedef float ntf4 __attribute__((ext_vector_type(4)));
+
+// the FP32 shadow of a state row (mixed path): the stage's gathers read it in place of the FP64 row
+DEV void ld4(const float4* p, uint32_t i, float o[4])
+{
+    const float4 t = p[i];
+    o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
+}
+DEV void st4(float4* p, uint32_t i, const float o[4]) { p[i] = make_float4(o[0], o[1], o[2], o[3]); }
+
+// ghost state from the owner state (solve.d:520-689); the owner is the only writer
+// false where the reference would stop: a total-conditions inflow with no non-negative Mach
+// root (solve.d:661-670)
+template <typename R>
+DEV bool ghostState(const BFace& b, const R qo[4], R qg[4], const R qgOld[4])
+{
+    const R g = R(G_), gm1 = R(G_ - 1), half = R(0.5), two = R(2.0);
+    switch (b.type) {
+    case BT_DIRICHLET:
+        qg[0] = R(b.gq[0]); qg[1] = R(b.gq[1]); qg[2] = R(b.gq[2]); qg[3] = R(b.gq[3]);
+        break;
+    case BT_INVWALL:
+    case BT_SYM: {
+        const R v0 = qo[1] / qo[0], v1 = qo[2] / qo[0];
+        R w0, w1;
+        if (!b.vertical) {
+            w0 = R(0.0) + R(b.R[0]) * v0 + R(b.R[1]) * v1;
+            w1 = R(0.0) + R(b.R[2]) * v0 + R(b.R[3]) * v1;
+        } else {
+            w0 = -v0;
+            w1 = v1;
+        }
+        qg[0] = qo[0]; qg[1] = qo[0] * w0; qg[2] = qo[0] * w1; qg[3] = qo[3];
+        break;
+    }
+    case BT_VISCWALL:
+        qg[0] = qo[0]; qg[1] = -qo[1]; qg[2] = -qo[2]; qg[3] = qo[3];
+        break;
+    case BT_CONSTP: {
+        const R rhop = qo[0], up = qo[1] / qo[0], vp = qo[2] / qo[0];
+        const R pp = pressure<R>(qo);
+        const R ap = sqrt(g * (pp / rhop));
+        const R Jp = up + (two * ap) / gm1;
+        const R Sp = pp / pow(rhop, g);
+        const R pb = R(b.data[0]);
+        const R rhob = pow(pb / Sp, R(1.0) / g);
+        const R ab = sqrt(g * (pb / rhob));
+        const R ub = Jp - (two * ab) / gm1;
+        const R vb = vp;
+        const R mag = sqrt(ub * ub + vb * vb);
+        const R rEb = pb / gm1 + half * rhob * (mag * mag);
+        const R n0 = R(b.nrm[0]), n1 = R(b.nrm[1]);
+        const R vpn = up * n0 + vp * n1, vbn = ub * n0 + vb * n1;
+        qg[0] = rhob;
+        qg[1] = rhob * (up - vpn * n0 + vbn * n0);
+        qg[2] = rhob * (vp - vpn * n1 + vbn * n1);
+        qg[3] = rEb;
+        break;
+    }
+    case BT_TPIN: {
+        // solve.d:625-683, including its four writes to component 0
+        const R Tt = R(b.data[0]), Pt = R(b.data[1]), ni0 = R(b.data[2]), ni1 = R(b.data[3]);
+        const R rhop = qo[0], up = qo[1] / qo[0];
+        const R pp = pressure<R>(qo);
+        const R ap = sqrt(g * (pp / rhop));
+        const R Jp = up + (two * ap) / gm1;
+        const R d = ni0 * R(b.nrm[0]) + ni1 * R(b.nrm[1]);
+        const R Rg = R(b.Rgas);
+        const R A = g * Rg * Tt * (d * d) - half * gm1 * (Jp * Jp);
+        const R B = (R(4.0) * g * Rg * Tt * d) / gm1;
+        const R Cc = (R(4.0) * g * Rg * Tt) / (gm1 * gm1) - Jp * Jp;
+        const R M1 = (-B + sqrt(B * B - R(4) * A * Cc)) / (two * A);
+        const R M2 = (-B - sqrt(B * B - R(4) * A * Cc)) / (two * A);
+        R Mb = R(NAN);
+        bool rootFound = true;
+        if (M1 >= 0 && M2 >= 0) Mb = fmin(M1, M2);
+        else if (M1 >= 0 && M2 < 0) Mb = M1;
+        else if (M1 < 0 && M2 >= 0) Mb = M2;
+        else rootFound = false;   // the reference stops here (enforce)
+        const R Tb = Tt / (R(1) + half * gm1 * (Mb * Mb));
+        const R pb = Pt * pow(Tb / Tt, g / gm1);
+        const R rhob = pb / (Rg * Tb);
+        const R ab = sqrt(g * (pb / rhob));
+        const R vb0 = Mb * ab * ni0, vb1 = Mb * ab * ni1;
+        const R mag = sqrt(vb0 * vb0 + vb1 * vb1);
+        qg[0] = pb / gm1 + half * rhob * (mag * mag);
+        qg[1] = qgOld[1]; qg[2] = qgOld[2]; qg[3] = qgOld[3];
+        return rootFound;
+    }
+    default:  // FullState
+        qg[0] = qo[0]; qg[1] = qo[1]; qg[2] = qo[2]; qg[3] = qo[3];
+        break;
+    }
+    return true;
+}
+
+// solve.d:27-173 LP vector limiter (all-inequality simplex, at most 16 pivots)
+DEV void lpSolve(int rows, const double* A, const double* b, const double c[2], double xk[2])
+{
+    int W0 = 0, W1 = 1;
+    double Ak[4] = {A[0], A[1], A[2], A[3]};
+    double gam[12];
+    int D[12];
+    for (int k = 0; k <= 15; k++) {
+        double det = Ak[0] * Ak[3] - Ak[1] * Ak[2];
+        double s = 1.0 / det;
+        const double iT0 = Ak[3] * s, iT1 = -Ak[2] * s, iT2 = -Ak[1] * s, iT3 = Ak[0] * s;
+        const double lam0 = 0.0 + iT0 * c[0] + iT1 * c[1];
+        const double lam1 = 0.0 + iT2 * c[0] + iT3 * c[1];
+        if ((lam0 >= -10e-9) && (lam1 >= -10e-9)) break;
+        const int q = (lam0 < lam1) ? W0 : W1;
+        const double e0 = (lam0 < lam1) ? 1.0 : 0.0, e1 = (lam0 < lam1) ? 0.0 : 1.0;
+        det = Ak[0] * Ak[3] - Ak[1] * Ak[2];
+        s = 1.0 / det;
+        const double i0 = Ak[3] * s, i1 = -Ak[1] * s, i2 = -Ak[2] * s, i3 = Ak[0] * s;
+        const double pk0 = 0.0 + i0 * e0 + i1 * e1;
+        const double pk1 = 0.0 + i2 * e0 + i3 * e1;
+        int Dlen = 0;
+        for (int i = 0; i < rows; i++)
+            if (i != W0 && i != W1)
+                if (A[2 * i] * pk0 + A[2 * i + 1] * pk1 < -1e-11) D[Dlen++] = i;
+        double alpha = INFINITY;
+        for (int i = 0; i < Dlen; i++) {
+            const double aixk = A[2 * D[i]] * xk[0] + A[2 * D[i] + 1] * xk[1];
+            const double aipk = A[2 * D[i]] * pk0 + A[2 * D[i] + 1] * pk1;
+            gam[i] = (aixk - b[D[i]]) / (-aipk);
+            alpha = fmin(alpha, gam[i]);
+        }
+        int t = 0;
+        for (int i = 0; i < Dlen; i++) if (gam[i] == alpha) { t = D[i]; break; }
+        if (q == W0) W0 = t; else if (q == W1) W1 = t;
+        Ak[0] = A[2 * W0]; Ak[1] = A[2 * W0 + 1]; Ak[2] = A[2 * W1]; Ak[3] = A[2 * W1 + 1];
+        xk[0] = xk[0] + alpha * pk0;
+        xk[1] = xk[1] + alpha * pk1;
+    }
+}
+
+// ---------------------------------------------------------------- gradient + limiter
+// solve.d:324-497 for one interior cell, given its own state, its S neighbour
+// states (ghosts already filled), LSQ weights, centroids and which slots are real
+// neighbours (padding slots repeat the cell).  MODE 1: unlimited; 2: scalar
+// limiter; 3: scalar limiter then the LP vector limiter.
+// Least-squares weights (A^T A)^-1 A^T with A_j = centroid_j - centroid_i, in the
+// operation order of the mesh set-up (source/mesh.d; mesh.cpp), so they equal the
+// stored ones bit for bit; the padding slots (A_j = 0) add exact zeros, as the
+// set-up's zero rows do.
+template <int S>
+DEV void lsqWeights(double2 ci, const double2 cn[S], double w[2][S])
+{
+    double ax[S], ay[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) { ax[j] = cn[j].x - ci.x; ay[j] = cn[j].y - ci.y; }
+    double b00 = 0.0, b01 = 0.0, b10 = 0.0, b11 = 0.0;
+#pragma unroll
+    for (int j = 0; j < S; j++) {
+        b00 += ax[j] * ax[j];
+        b01 += ax[j] * ay[j];
+        b10 += ay[j] * ax[j];
+        b11 += ay[j] * ay[j];
+    }
+    const double det = b00 * b11 - b01 * b10;
+    const double id = 1.0 / det;
+    const double i00 = b11 * id, i01 = -b01 * id, i10 = -b10 * id, i11 = b00 * id;
+#pragma unroll
+    for (int j = 0; j < S; j++) {
+        w[0][j] = i00 * ax[j] + i01 * ay[j];
+        w[1][j] = i10 * ax[j] + i11 * ay[j];
+    }
+}
+
+// gm: stored weights ((dir, nbr)-major, stride gstride between entries), or null
+// to compute them from the centroids.  Weights and centroid offsets are geometry,
+// computed in FP64 and converted to R; the gradient, bounds and limiter are R.
+// MODE 4: the Venkatakrishnan limiter at the same test points (neighbour centroids): for
+// the unlimited increment t = grad . (x_j - x_i) and the bound difference d = max - q_i (t > 0)
+// or min - q_i (t < 0), phi_j = [(d^2 + eps2) t + 2 t^2 d] / (t [d^2 + 2 t^2 + d t + eps2]),
+// phi = min(1, min_j phi_j); eps2 = (K d_cell)^3 (FP64, passed in).
+template <int S, int MODE, typename R>
+DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t gstride, double2 ci,
+                   const double2 cn[S], const bool real[S], int limit, double lpThresh, R g[4][2], R lx[4],
+                   R ly[4], double eps2d = 0.0)
+{
+    static_assert(MODE != 3 || sizeof(R) == 8, "the LP vector limiter runs in FP64 only");
+    R w[2][S];
+    {
+        double wd[2][S];
+        if (gm) {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int j = 0; j < S; j++) wd[r][j] = gm[(r * S + j) * gstride];
+        } else {
+            lsqWeights<S>(ci, cn, wd);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int j = 0; j < S; j++) w[r][j] = R(wd[r][j]);
+    }
+    R mn[4], mx[4], du[4][S];
+#pragma unroll
+    for (int k = 0; k < 4; k++) { mn[k] = qi[k]; mx[k] = qi[k]; }
+#pragma unroll
+    for (int j = 0; j < S; j++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            mn[k] = fmin(mn[k], qn[j][k]);
+            mx[k] = fmax(mx[k], qn[j][k]);
+            du[k][j] = qn[j][k] - qi[k];
+        }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            R s = R(0.0);
+#pragma unroll
+            for (int j = 0; j < S; j++) s += w[r][j] * du[k][j];
+            g[k][r] = s;
+        }
+#pragma unroll
+    for (int k = 0; k < 4; k++) { lx[k] = R(1.0); ly[k] = R(1.0); }
+    if (MODE == 4 && limit) {
+        const R eps2 = R(eps2d), two = R(2.0);
+#pragma unroll
+        for (int j = 0; j < S; j++) {
+            const R dx = R(cn[j].x - ci.x), dy = R(cn[j].y - ci.y);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const R t = g[k][0] * dx + g[k][1] * dy;
+                R s = R(1.0);
+                if (t != R(0.0)) {
+                    const R d = t > R(0.0) ? mx[k] - qi[k] : mn[k] - qi[k];
+                    s = ((d * d + eps2) * t + two * (t * t) * d) / (t * (d * d + two * (t * t) + d * t + eps2));
+                }
+                lx[k] = fmin(lx[k], s);
+                ly[k] = lx[k];
+            }
+        }
+        return;
+    }
+    if (MODE >= 2 && MODE <= 3 && limit) {
+        R dxs[S], dys[S];
+#pragma unroll
+        for (int j = 0; j < S; j++) {
+            const R dx = R(cn[j].x - ci.x), dy = R(cn[j].y - ci.y);
+            dxs[j] = dx; dys[j] = dy;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                R s = R(1.0);
+                const R t = g[k][0] * dx + g[k][1] * dy;
+                const R qE = qi[k] + t;
+                if (qE < mn[k]) s = (mn[k] - qi[k]) / t;
+                else if (qE > mx[k]) s = (mx[k] - qi[k]) / t;
+                lx[k] = fmin(lx[k], s);
+                ly[k] = lx[k];
+            }
+        }
+        if constexpr (MODE == 3) {
+            if (lpThresh > 0) {
+                int nn = 0;
+#pragma unroll
+                for (int j = 0; j < S; j++) nn += real[j] ? 1 : 0;
+                for (int k = 0; k < 4; k++) {
+                    if (lx[k] < lpThresh && (nn == 3 || nn == 4)) {
+                        double A[24], bb[12];
+                        for (int r = 0; r < 24; r++) A[r] = 0.0;
+                        for (int r = 0; r < 12; r++) bb[r] = 0.0;
+                        A[0] = 1; A[3] = 1; A[4] = -1; A[7] = -1;
+                        bb[2] = -1; bb[3] = -1;
+                        int c2 = 0;
+                        for (int j = 0; j < S; j++) {
+                            if (!real[j]) continue;
+                            A[2 * (c2 + 4)] = dxs[j] * g[k][0];
+                            A[2 * (c2 + 4) + 1] = dys[j] * g[k][1];
+                            bb[c2 + 4] = mn[k] - qi[k];
+                            A[2 * (c2 + 5)] = -dxs[j] * g[k][0];
+                            A[2 * (c2 + 5) + 1] = -dys[j] * g[k][1];
+                            bb[c2 + 5] = qi[k] - mx[k];
+                            c2 += 2;
+                        }
+                        const double cc[2] = {-fabs(g[k][0]), -fabs(g[k][1])};
+                        double xk[2] = {0.0, 0.0};
+                        lpSolve(4 + 2 * nn, A, bb, cc, xk);
+                        lx[k] = xk[0];
+                        ly[k] = xk[1];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// the owner's ghost state for boundary record b, with TempPresInflow's untouched components
+DEV bool ghostFromOwner(const BFace& bf, const double qo[4], const double4* qbuf, uint32_t gIdx, double qg[4])
+{
+    double old[4] = {0, 0, 0, 0};
+    if (bf.type == BT_TPIN) ld4(qbuf, gIdx, old);
+    return ghostState(bf, qo, qg, old);
+}
+
+// The boundary force sum of mesh.d:645-671: (len*flux) momentum components of the
+// force faces added in order, two interleaved chains, by thread 0 (its result).
+// fp: LDS staging of CAP (x, y) pairs.
+template <int NT, int CAP>
+DEV void orderedForce(const uint32_t* faces, uint32_t nF, const double* lenF, double2* fp, double& f0, double& f1)
+{
+    f0 = 0; f1 = 0;
+    for (uint32_t k0 = 0; k0 < nF; k0 += CAP) {
+        const uint32_t cnt = (nF - k0) < uint32_t(CAP) ? (nF - k0) : uint32_t(CAP);
+        __syncthreads();
+        // all of a thread's face ids, then all of their fluxes, are loaded before any is
+        // used: two round trips per pass instead of two per face
+        constexpr int FS = (CAP + NT - 1) / NT;
+        uint32_t fi[FS];
+#pragma unroll
+        for (int u = 0; u < FS; u++) {
+            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
+            fi[u] = x < cnt ? faces[k0 + x] : 0u;
+        }
+        double2 fv[FS];
+#pragma unroll
+        for (int u = 0; u < FS; u++) {
+            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
+            fv[u] = x < cnt ? make_double2(lenF[size_t(fi[u]) * 4 + 1], lenF[size_t(fi[u]) * 4 + 2])
+                            : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int u = 0; u < FS; u++) {
+            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
+            if (x < cnt) fp[x] = fv[u];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            // the two ordered chains interleave; 32 LDS reads are in flight ahead of the adds
+            uint32_t x = 0;
+            for (; x + 32 <= cnt; x += 32) {
+                double2 v[32];
+#pragma unroll
+                for (int u = 0; u < 32; u++) v[u] = fp[x + u];
+#pragma unroll
+                for (int u = 0; u < 32; u++) { f0 += v[u].x; f1 += v[u].y; }
+            }
+            for (; x < cnt; x++) { const double2 v = fp[x]; f0 += v.x; f1 += v.y; }
+        }
+    }
+}
+
+// a pending force (k_finalize left it): rotated drag/lift into the step's history row
+// and the scalars, as k_finalize would have written them
+template <int NT, int CAP>
+DEV void pendingForce(const ForceArgs& f, DevScalars* sc, double2* fp)
+{
+    if (!sc->forcePending) return;
+    double f0, f1;
+    orderedForce<NT, CAP>(f.faces, f.n, f.lenF, fp, f0, f1);
+    if (threadIdx.x == 0) {
+        const double ld0 = 0.0 + f.rot[0] * f0 + f.rot[1] * f1;
+        const double ld1 = 0.0 + f.rot[2] * f0 + f.rot[3] * f1;
+        const int64_t slot = sc->forceSlot;
+        if (slot >= 0) {
+            double* h = f.hist + slot * HIST_FIELDS;
+            h[7] = ld0; h[8] = ld1;
+        }
+        sc->force[0] = ld0; sc->force[1] = ld1;
+        sc->forcePending = 0;
+    }
+}
+
+// MODE 0: ghost states only (order 1); 1: unlimited gradient (no limiter stored);
+// 2: scalar limiter; 3: scalar limiter followed by the LP vector limiter (lim
+// stored as x,y pairs).
+// MIX 0: FP64 throughout.  MIX 1 (mixed precision): states are read from the FP32
+// shadows, ghosts, gradients and limiters computed in FP32 (least-squares weights and
+// centroid offsets in FP64, converted); gradients and limiters are stored as FP32
+// rows (32 + 16 bytes per cell); each ghost is written to the shadow and, widened, to
+// the FP64 row.
+// LDS of one gradient workgroup: staging of the gradient rows (and of the force faces)
+// and of the limiter rows
+template <int MODE>
+struct GradLds {
+    static constexpr int LWS = MODE == 3 ? 8 : ((MODE == 2 || MODE == 4) ? 4 : 0);
+    double sg[BLK][9];
+    double sl[BLK][LWS + 1];
+};
+
+template <int MIX>
+using RealOf = typename std::conditional<MIX == 1, float, double>::type;
+
+// a stage-input row: the FP32 shadow on the mixed path
+template <int MIX>
+DEV void ldStage(const StageArgs& a, uint32_t c, RealOf<MIX> o[4])
+{
+    if constexpr (MIX == 1) ld4(a.qin32, c, o);
+    else ld4(a.qin, c, o);
+}
+// a ghost row of the stage input; the mixed path also widens it into the FP64 row
+template <int MIX>
+DEV void stGhostRow(const StageArgs& a, uint32_t c, const RealOf<MIX> o[4])
+{
+    if constexpr (MIX == 1) {
+        st4(a.qin32, c, o);
+        a.qin[c] = make_double4(o[0], o[1], o[2], o[3]);
+    } else {
+        st4(a.qin, c, o);
+    }
+}
+
+// Gradient and limiter of interior cell i (MODE 1-4) from the stage input, with the ghost
+// states of its boundary faces, which are stored to the stage buffer where storeGhosts;
+// nbrRow: its S neighbour ids (the mesh's row, or a tile's copy of it).
+// Every neighbour row is loaded before any ghost is written, so the loads of all
+// neighbours are in flight together.  A ghost slot belongs to this cell alone (the owner of
+// its boundary face), so its row still holds the stage buffer's previous ghost state, which
+// TempPresInflow keeps in the components it does not write.
+template <int S, int MODE, int MIX>
+DEV void cellGradient(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t i, const uint32_t* nbrRow,
+                      bool storeGhosts, RealOf<MIX> g[4][2], RealOf<MIX> lx[4], RealOf<MIX> ly[4])
+{
+    using R = RealOf<MIX>;
+    R qi[4];
+    ldStage<MIX>(a, i, qi);
+    uint32_t nb[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) nb[j] = nbrRow[j];
+    R qn[S][4];
+    double2 cn[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) { ldStage<MIX>(a, nb[j], qn[j]); cn[j] = m.cen[nb[j]]; }
+    const double2 ci = m.cen[i];
+#pragma unroll
+    for (int j = 0; j < S; j++)
+        if (nb[j] >= m.N) {
+            const BFace& bf = m.bface[nb[j] - m.N];
+            R old[4] = {0, 0, 0, 0};
+            if (bf.type == BT_TPIN) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) old[k] = qn[j][k];
+            }
+            if (!ghostState<R>(bf, qi, qn[j], old) && a.recordErrors)
+                atomicMin(&a.sc->errBC, (uint64_t(a.stageId) << 32) | (nb[j] - m.N));
+            if (storeGhosts) stGhostRow<MIX>(a, nb[j], qn[j]);
+        }
+    bool real[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) real[j] = nb[j] != i;
+    double eps2 = 0.0;
+    if constexpr (MODE == 4) {
+        const double kd = p.venkatK * m.cd[i];
+        eps2 = kd * kd * kd;
+    }
+    gradLimit<S, MODE, R>(qi, qn, nullptr, 0, ci, cn, real, a.limit, p.lpThresh, g, lx, ly, eps2);
+}
+
+// One workgroup of the gradient kernel on cell block `bid` of its mesh (the solo and the
+// batched kernels run this same code).
+template <int S, int MODE, int MIX>
+DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid, GradLds<MODE>& L)
+{
+    using R = RealOf<MIX>;
+    constexpr int LWS = GradLds<MODE>::LWS;
+    auto& sg = L.sg;
+    auto& sl = L.sl;
+    if (a.checkActive && !a.sc->active) return;
+    if (bid == 0 && threadIdx.x == 0 && a.first) a.sc->rmaxBits = 0;   // Rmax is per step
+    const uint32_t i = bid * BLK + threadIdx.x;
+    if (MODE == 0 && i >= m.N) return;
+    const bool have = i < m.N;   // no early return below: the staged stores need every thread
+    R g[4][2], lx[4], ly[4];
+    if (have) {
+        if constexpr (MODE == 0) {
+            // order 1: the ghost states are the kernel's only output
+            R qi[4];
+            ldStage<MIX>(a, i, qi);
+#pragma unroll
+            for (int j = 0; j < S; j++) {
+                const uint32_t nb = m.nbr[i * S + j];
+                if (nb >= m.N) {
+                    const BFace& bf = m.bface[nb - m.N];
+                    R qg[4], old[4] = {0, 0, 0, 0};
+                    if (bf.type == BT_TPIN) ldStage<MIX>(a, nb, old);
+                    if (!ghostState<R>(bf, qi, qg, old) && a.recordErrors)
+                        atomicMin(&a.sc->errBC, (uint64_t(a.stageId) << 32) | (nb - m.N));
+                    stGhostRow<MIX>(a, nb, qg);
+                }
+            }
+            return;
+        } else {
+            cellGradient<S, MODE, MIX>(m, p, a, i, m.nbr + size_t(i) * S, true, g, lx, ly);
+        }
+    }
+    if (MODE == 0) return;
+    // stage the rows in LDS and store the workgroup's contiguous run of cells with
+    // lane-consecutive 16-byte stores
+    const uint32_t tid = threadIdx.x;
+    const uint32_t base = bid * BLK, n = (m.N - base) < BLK ? (m.N - base) : BLK;
+    if constexpr (MIX == 1) {
+        float* fg = reinterpret_cast<float*>(&sg[0][0]);   // 8 floats per row
+        float* fl = reinterpret_cast<float*>(&sl[0][0]);   // 4 floats per row
+        if (have) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) { fg[8 * tid + 2 * c] = g[c][0]; fg[8 * tid + 2 * c + 1] = g[c][1]; }
+            if (MODE == 2 || MODE == 4) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) fl[4 * tid + c] = lx[c];
+            }
+        }
+        __syncthreads();
+        float4* gd = reinterpret_cast<float4*>(a.grad32 + size_t(base) * 8);
+        for (uint32_t c = tid; c < 2 * n; c += BLK)
+            __builtin_nontemporal_store(*reinterpret_cast<const ntf4*>(fg + 4 * c), reinterpret_cast<ntf4*>(gd) + c);
+        if (MODE == 2 || MODE == 4) {
+            float4* ld = reinterpret_cast<float4*>(a.lim32 + size_t(base) * 4);
+            for (uint32_t c = tid; c < n; c += BLK)
+                __builtin_nontemporal_store(*reinterpret_cast<const ntf4*>(fl + 4 * c), reinterpret_cast<ntf4*>(ld) + c);
+        }
+        return;
+    } else {
+        if (have) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) { sg[tid][2 * c] = g[c][0]; sg[tid][2 * c + 1] = g[c][1]; }
+            if (MODE == 3) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) { sl[tid][2 * c] = lx[c]; sl[tid][2 * c + 1] = ly[c]; }
+            } else if (MODE == 2 || MODE == 4) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) sl[tid][c] = lx[c];
+            }
+        }
+        __syncthreads();
+        double2* gd = reinterpret_cast<double2*>(a.grad + size_t(base) * 8);
+        for (uint32_t c = tid; c < 4 * n; c += BLK) __builtin_nontemporal_store((ntd2){sg[c / 4][2 * (c % 4)], sg[c / 4][2 * (c % 4) + 1]}, reinterpret_cast<ntd2*>(gd) + c);
+        if constexpr (LWS > 0) {
+            double2* ld = reinterpret_cast<double2*>(a.lim + size_t(base) * LWS);
+            constexpr uint32_t PR = LWS / 2;
+            for (uint32_t c = tid; c < PR * n; c += BLK) __builtin_nontemporal_store((ntd2){sl[c / PR][2 * (c % PR)], sl[c / PR][2 * (c % PR) + 1]}, reinterpret_cast<ntd2*>(ld) + c);
+        }
+    }
+    // MODE 1 (unlimited stage): every limiter is 1; the face kernels take LP = 2 and read none
+}
+// ---------------------------------------------------------------- faces
+// LP 0: scalar limiter (4 per cell); 1: LP vector limiter (x,y pairs); 2: an
+// unlimited stage, every limiter 1 (1*g is exactly g, so the products round as with
+// stored ones)
+template <int LP>
+DEV void loadLim(const double* lim, uint32_t c, double lx[4], double ly[4])
+{
+    if (LP == 2) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) { lx[k] = 1.0; ly[k] = 1.0; }
+    } else if (LP) {
+        const double4 a = *reinterpret_cast<const double4*>(lim + size_t(c) * 8);
+        const double4 b = *reinterpret_cast<const double4*>(lim + size_t(c) * 8 + 4);
+        lx[0] = a.x; ly[0] = a.y; lx[1] = a.z; ly[1] = a.w; lx[2] = b.x; ly[2] = b.y; lx[3] = b.z; ly[3] = b.w;
+    } else {
+        const double4 a = *reinterpret_cast<const double4*>(lim + size_t(c) * 4);
+        lx[0] = ly[0] = a.x; lx[1] = ly[1] = a.y; lx[2] = ly[2] = a.z; lx[3] = ly[3] = a.w;
+    }
+}
+// FP32 rows of the mixed path (no LP vector limiter there)
+template <int LP>
+DEV void loadLim(const float* lim, uint32_t c, float lx[4], float ly[4])
+{
+    static_assert(LP != 1, "the LP vector limiter runs in FP64 only");
+    if (LP == 2) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) { lx[k] = 1.0f; ly[k] = 1.0f; }
+    } else {
+        const float4 a = *reinterpret_cast<const float4*>(lim + size_t(c) * 4);
+        lx[0] = ly[0] = a.x; lx[1] = ly[1] = a.y; lx[2] = ly[2] = a.z; lx[3] = ly[3] = a.w;
+    }
+}
+
+DEV void loadGrad(const double* grad, uint32_t c, double g[8])
+{
+    const double4 a = *reinterpret_cast<const double4*>(grad + size_t(c) * 8);
+    const double4 b = *reinterpret_cast<const double4*>(grad + size_t(c) * 8 + 4);
+    g[0] = a.x; g[1] = a.y; g[2] = a.z; g[3] = a.w; g[4] = b.x; g[5] = b.y; g[6] = b.z; g[7] = b.w;
+}
+DEV void loadGrad(const float* grad, uint32_t c, float g[8])
+{
+    const float4 a = *reinterpret_cast<const float4*>(grad + size_t(c) * 8);
+    const float4 b = *reinterpret_cast<const float4*>(grad + size_t(c) * 8 + 4);
+    g[0] = a.x; g[1] = a.y; g[2] = a.z; g[3] = a.w; g[4] = b.x; g[5] = b.y; g[6] = b.z; g[7] = b.w;
+}
+
+// solve.d:980-1010 (interior) reconstruction with the p<0 fallback
+template <int LP, typename R>
+DEV void reconstruct(const R qm[4], const R g[8], const R lx[4], const R ly[4], R dx, R dy, R out[4])
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) out[j] = qm[j] + lx[j] * g[2 * j] * dx + ly[j] * g[2 * j + 1] * dy;
+    if (pressure<R>(out) < 0) {
+        R l0 = R(1.0), l1 = R(1.0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) { l0 = fmin(l0, lx[j]); l1 = fmin(l1, ly[j]); }
+#pragma unroll
+        for (int j = 0; j < 4; j++) out[j] = qm[j] + l0 * g[2 * j] * dx + l1 * g[2 * j + 1] * dy;
+    }
+}
+
+// solve.d:970-1033: one interior face from both cells' raw data.  Centroids, midpoint
+// and normal are FP64 geometry; the offsets and the normal enter the R arithmetic.
+template <int FLUX, int VISC, int ORDER, int LP, typename R>
+DEV void interiorFace(const R qa[4], const R ga[8], const R lxa[4], const R lya[4], double2 ca,
+                      const R qb[4], const R gb[8], const R lxb[4], const R lyb[4], double2 cb,
+                      double2 n, double2 mid, const PhysParams& p, R qL[4], R qR[4], R F[4], R& sMax)
+{
+    if (ORDER > 1) {
+        reconstruct<LP, R>(qa, ga, lxa, lya, R(mid.x - ca.x), R(mid.y - ca.y), qL);
+        reconstruct<LP, R>(qb, gb, lxb, lyb, R(mid.x - cb.x), R(mid.y - cb.y), qR);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) { qL[k] = qa[k]; qR[k] = qb[k]; }
+    }
+    // the face gradient is formed before the convective flux, so the two cell gradients
+    // are not live across it
+    R dq[8];
+    if (VISC) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) dq[k] = R(0.5) * (ga[k] + gb[k]);
+    }
+    numFlux<FLUX, R>(qL, qR, R(n.x), R(n.y), F, sMax);
+    if (VISC) {
+        R qa2[4], Fv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) qa2[k] = R(0.5) * (qL[k] + qR[k]);
+        viscousFlux<R>(p.Pr, p.mu, qa2, dq, R(n.x), R(n.y), Fv);
+#pragma unroll
+        for (int k = 0; k < 4; k++) F[k] = F[k] - Fv[k];
+    }
+}
+
+// solve.d:283-319 + 769-968: one boundary face from its owner's data and ghost state
+template <int FLUX, int VISC, int ORDER, int LP, typename R>
+DEV void boundaryFace(const R qo[4], const R gO[8], const R lx[4], const R ly[4], double2 co,
+                      const R qg[4], const BFace& bf, double2 nd, double2 mid, const PhysParams& p,
+                      R qL[4], R qR[4], R F[4], R& sMax)
+{
+    const R g = R(G_), gm1 = R(G_ - 1), half = R(0.5);
+    const R nx = R(nd.x), ny = R(nd.y);
+    // updateBoundaryEdge: the fallback uses lim[0] for both directions
+    if (ORDER > 1) {
+        const R dx = R(mid.x - co.x), dy = R(mid.y - co.y);
+#pragma unroll
+        for (int j = 0; j < 4; j++) qL[j] = qo[j] + lx[j] * gO[2 * j] * dx + ly[j] * gO[2 * j + 1] * dy;
+        if (pressure<R>(qL) < 0) {
+            R l0 = R(1.0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) l0 = fmin(l0, lx[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) qL[j] = qo[j] + l0 * gO[2 * j] * dx + l0 * gO[2 * j + 1] * dy;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) qL[j] = qo[j];
+    }
+    const int type = bf.type;
+    if (type == BT_FULL || type == BT_DIRICHLET) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) qR[k] = R(bf.far[k]);
+        numFlux<FLUX, R>(qL, qR, nx, ny, F, sMax);
+        if (VISC) {
+            R qa[4], dq[8], Fv[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) qa[k] = half * (qL[k] + qR[k]);
+            if (type == BT_DIRICHLET) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) dq[k] = half * (gO[k] + R(bf.gg[k]));
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; k++) dq[k] = half * (gO[k] + R(0.0));
+            }
+            viscousFlux<R>(p.Pr, p.mu, qa, dq, nx, ny, Fv);
+#pragma unroll
+            for (int k = 0; k < 4; k++) F[k] = F[k] - Fv[k];
+        }
+    } else if (type == BT_INVWALL) {
+        const R inv = R(1) / qL[0];
+        const R v0 = inv * qL[1], v1 = inv * qL[2];
+        const R vn = v0 * nx + v1 * ny;
+        const R t0 = v0 - vn * nx, t1 = v1 - vn * ny;
+        const R vel = sqrt(t0 * t0 + t1 * t1);
+        R pw = gm1 * (qL[3] - half * qL[0] * (vel * vel));
+        const R aw = sqrt(g * (pw / qL[0]));
+        if (pw < 0) pw = R(1.0e-12);
+        F[0] = R(0); F[1] = pw * nx; F[2] = pw * ny; F[3] = R(0);
+        sMax = fabs(aw);
+        for (int k = 0; k < 4; k++) qR[k] = qg[k];
+    } else if (type == BT_VISCWALL) {
+        const R vel = R(0.0);
+        R pw = gm1 * (qL[3] - half * qL[0] * (vel * vel));
+        const R aw = sqrt(g * (pw / qL[0]));
+        if (pw < 0) pw = R(1.0e-12);
+        qR[0] = qL[0]; qR[1] = qL[1] * R(-1); qR[2] = qL[2] * R(-1); qR[3] = qL[3];
+        R qa[4], dq[8], Fv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) qa[k] = half * (qL[k] + qR[k]);
+        qa[1] = R(0.0); qa[2] = R(0.0);
+#pragma unroll
+        for (int k = 0; k < 8; k++) dq[k] = gO[k];
+        dq[6] = (qa[3] / qa[0]) * dq[0];
+        dq[7] = (qa[3] / qa[0]) * dq[1];
+        viscousFlux<R>(p.Pr, p.mu, qa, dq, nx, ny, Fv);
+        F[0] = R(0) - Fv[0]; F[1] = pw * nx - Fv[1]; F[2] = pw * ny - Fv[2]; F[3] = R(0) - Fv[3];
+        sMax = fabs(aw);
+    } else if (type == BT_CONSTP) {
+        for (int k = 0; k < 4; k++) qR[k] = qg[k];
+        const R pg = pressure<R>(qR);
+        const R ug = qR[1] / qR[0], vg = qR[2] / qR[0];
+        const R ag = sqrt(g * (pg / qR[0]));
+        convective<R>(pg, ug, vg, qR[0], qR[3], nx, ny, F);
+        sMax = fabs(ag);
+    } else if (type == BT_SYM) {
+        const R v0 = qL[1] / qL[0], v1 = qL[2] / qL[0];
+        R w0, w1;
+        if (!bf.vertical) {
+            w0 = R(0.0) + R(bf.R[0]) * v0 + R(bf.R[1]) * v1;
+            w1 = R(0.0) + R(bf.R[2]) * v0 + R(bf.R[3]) * v1;
+        } else {
+            w0 = -v0;
+            w1 = v1;
+        }
+        qR[0] = qL[0]; qR[1] = qL[0] * w0; qR[2] = qL[0] * w1; qR[3] = qL[3];
+        numFlux<FLUX, R>(qL, qR, nx, ny, F, sMax);
+        if (VISC) {
+            const R one = R(1), zero = R(0), two = R(2);
+            R qa[4], bg[8], Fv[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) qa[k] = half * (qL[k] + qR[k]);
+            const R o00 = nx * nx, o01 = nx * ny, o10 = ny * nx, o11 = ny * ny;
+            const R V00 = one - o00, V01 = zero - o01, V10 = zero - o10, V11 = one - o11;
+            const R T00 = one - two * o00, T01 = zero - two * o01, T10 = zero - two * o10, T11 = one - two * o11;
+            // tmp1 = A*gradp with A = identity except the momentum block V (4x4 * 4x2, all columns)
+            R t1[8];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                t1[0 + c] = zero + one * gO[0 + c] + zero * gO[2 + c] + zero * gO[4 + c] + zero * gO[6 + c];
+                t1[2 + c] = zero + zero * gO[0 + c] + V00 * gO[2 + c] + V01 * gO[4 + c] + zero * gO[6 + c];
+                t1[4 + c] = zero + zero * gO[0 + c] + V10 * gO[2 + c] + V11 * gO[4 + c] + zero * gO[6 + c];
+                t1[6 + c] = zero + zero * gO[0 + c] + zero * gO[2 + c] + zero * gO[4 + c] + one * gO[6 + c];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const R s30 = zero + t1[2 * r] * T00 + t1[2 * r + 1] * T10;
+                const R s31 = zero + t1[2 * r] * T01 + t1[2 * r + 1] * T11;
+                const R s10 = zero + gO[2 * r] * o00 + gO[2 * r + 1] * o10;
+                const R s11 = zero + gO[2 * r] * o01 + gO[2 * r + 1] * o11;
+                bg[2 * r] = s10 + s30;
+                bg[2 * r + 1] = s11 + s31;
+            }
+            viscousFlux<R>(p.Pr, p.mu, qa, bg, nx, ny, Fv);
+#pragma unroll
+            for (int k = 0; k < 4; k++) F[k] = F[k] - Fv[k];
+        }
+    } else {  // TempPresInflow
+        for (int k = 0; k < 4; k++) qR[k] = qg[k];
+        numFlux<FLUX, R>(qL, qR, nx, ny, F, sMax);
+        if (VISC) {
+            R qa[4], Fv[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) qa[k] = half * (qL[k] + qR[k]);
+            viscousFlux<R>(p.Pr, p.mu, qa, gO, nx, ny, Fv);
+#pragma unroll
+            for (int k = 0; k < 4; k++) F[k] = F[k] - Fv[k];
+        }
+    }
+}
+
+// Cell data a face reads: the FP64 rows, or on the mixed path (MIX 1) the FP32
+// shadow of the state and the FP32 gradient and limiter rows.
+template <int MIX>
+struct FaceSrc {
+    using R = typename std::conditional<MIX == 1, float, double>::type;
+    const StageArgs& a;
+    DEV void q(uint32_t c, R o[4]) const
+    {
+        if constexpr (MIX == 1) ld4(a.qin32, c, o);
+        else ld4(a.qin, c, o);
+    }
+    DEV void grad(uint32_t c, R o[8]) const
+    {
+        if constexpr (MIX == 1) loadGrad(a.grad32, c, o);
+        else loadGrad(a.grad, c, o);
+    }
+    template <int LP>
+    DEV void lim(uint32_t c, R lx[4], R ly[4]) const
+    {
+        if constexpr (MIX == 1) loadLim<LP>(a.lim32, c, lx, ly);
+        else loadLim<LP>(a.lim, c, lx, ly);
+    }
+};
+
+// ---------------------------------------------------------------- residual + update
+DEV double warpMin(double v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
+    return v;
+}
+DEV double warpMax(double v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// solve.d:1092-1117 + the integrator's stage update for interior cell i, from
+// its summed face fluxes r and sum of len*sMax
+// met: (perimeter, d, -1/area) of the cell, or null to read them from the mesh
+// qNew/qOld (optional): the new state and q^n when this stage completes a step
+// qnI, accI (optional): the cell's q^n and RK accumulator rows already loaded
+// the stage output row, and on the mixed path its FP32 shadow for the next stage's gathers
+DEV void storeOut(const StageArgs& a, uint32_t i, const double o[4])
+{
+    st4(a.qout, i, o);
+    if (a.qout32) a.qout32[i] = make_float4(float(o[0]), float(o[1]), float(o[2]), float(o[3]));
+}
+
+template <int KIND>
+DEV void cellStage(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t i, const double r[4],
+                   double sAve, const double* qinI, const double* met, double& dtCand, double& rCand,
+                   double* qNew = nullptr, double* qOld = nullptr, const double* qnI = nullptr,
+                   const double* accI = nullptr)
+{
+    auto loadAcc = [&](double v[4]) {
+        if (accI) { v[0] = accI[0]; v[1] = accI[1]; v[2] = accI[2]; v[3] = accI[3]; }
+        else ld4(a.acc, i, v);
+    };
+    const double cper = met ? met[0] : m.cper[i], cd = met ? met[1] : m.cd[i], nia = met ? met[2] : m.nia[i];
+    sAve /= cper;
+    const double CFL = a.sc->CFL;
+    const double dtc = (CFL * cd) / sAve;
+    if (!isnan(dtc)) dtCand = fmin(dtCand, dtc);
+    double hc = 0.0;
+    if (p.localTimestep) {
+        if (a.dtUpdate) {
+            hc = CFL * cd / sAve;
+            if (isnan(hc)) hc = 0;
+            a.celldt[i] = hc;
+        } else {
+            hc = a.celldt[i];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) if (fabs(r[k]) > rCand) rCand = fabs(r[k]);
+    const double s = nia;
+    double R[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) R[k] = r[k] * s;
+    if (m.src) {
+        const double4 sv = m.src[i];
+        R[0] = R[0] + sv.x; R[1] = R[1] + sv.y; R[2] = R[2] + sv.z; R[3] = R[3] + sv.w;
+    }
+    const double dt = a.sc->dt;
+    const double h = p.localTimestep ? hc : dt;
+    double qn[4], o[4];
+    if (KIND != SK_RESIDUAL) {
+        if (qnI) { qn[0] = qnI[0]; qn[1] = qnI[1]; qn[2] = qnI[2]; qn[3] = qnI[3]; }
+        else ld4(a.qn, i, qn);
+    }
+    if (KIND == SK_RESIDUAL) {
+        st4(a.R, i, R);
+    } else if (KIND == SK_EULER) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + h * R[k];
+        storeOut(a, i, o);
+    } else if (KIND == SK_RK2_1) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + (dt * R[k]);
+        st4(a.acc, i, R);
+        storeOut(a, i, o);
+    } else if (KIND == SK_RK2_2) {
+        double k1[4];
+        loadAcc(k1);
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + (h / 2.0) * (k1[k] + R[k]);
+        storeOut(a, i, o);
+    } else if (KIND == SK_TVD_1) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + h * R[k];
+        storeOut(a, i, o);
+    } else if (KIND == SK_TVD_2) {
+        double fe[4];
+        if (qinI) { fe[0] = qinI[0]; fe[1] = qinI[1]; fe[2] = qinI[2]; fe[3] = qinI[3]; }
+        else ld4(a.qin, i, fe);
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = 0.5 * (qn[k] + fe[k] + h * R[k]);
+        storeOut(a, i, o);
+    } else if (KIND == SK_RK4_1) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + ((dt / 2.0) * R[k]);
+        st4(a.acc, i, R);
+        storeOut(a, i, o);
+    } else if (KIND == SK_RK4_2 || KIND == SK_RK4_3) {
+        double ac[4];
+        loadAcc(ac);
+#pragma unroll
+        for (int k = 0; k < 4; k++) ac[k] = ac[k] + 2.0 * R[k];
+        const double c = (KIND == SK_RK4_2) ? (dt / 2.0) : dt;
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + (c * R[k]);
+        st4(a.acc, i, ac);
+        storeOut(a, i, o);
+    } else if (KIND == SK_RK4_4) {
+        double ac[4];
+        loadAcc(ac);
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = qn[k] + (h / 6.0) * (ac[k] + R[k]);
+        storeOut(a, i, o);
+    }
+    if (KIND != SK_RESIDUAL && a.last && a.recordErrors &&
+        (isnan(o[0]) || isnan(o[1]) || isnan(o[2]) || isnan(o[3])))
+        atomicMin(&a.sc->errCell, (uint64_t(a.stepId) << 32) | m.refId[i]);
+    if ((KIND == SK_EULER || KIND == SK_RK2_2 || KIND == SK_TVD_2 || KIND == SK_RK4_4) && qNew) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) { qNew[k] = o[k]; qOld[k] = qn[k]; }
+    }
+}
+
+// Leaf sums of the RMS residual's pairwise sum (app/solver.d:153-168), fused into
+// the stage that completes a step.  Each group of 16 lanes holds one aligned block
+// of 16 consecutive reference cells, lane j its element j (absent cells add
+// zeros); the xor butterfly adds exactly like the fixed 16-element tree, and lane
+// 0 of the group stores the block's 8 sums: (new - old)^2 and new per variable.
+// Every lane of the wave must call this.
+DEV void rmsBlockLeaf(bool have, const double qNew[4], const double qOld[4], uint32_t refCell, double* rmsBlocks)
+{
+    double o[8];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const double x = have ? qNew[v] - qOld[v] : 0.0;
+        o[v] = have ? x * x : 0.0;
+        o[4 + v] = have ? qNew[v] : 0.0;
+    }
+#pragma unroll
+    for (int mm = 1; mm < 16; mm <<= 1)
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = o[q] + __shfl_xor(o[q], mm, 64);
+    if (have && (threadIdx.x & 15u) == 0) {
+        double* dst = rmsBlocks + size_t(refCell / 16) * 8;
+        *reinterpret_cast<double4*>(dst) = make_double4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<double4*>(dst + 4) = make_double4(o[4], o[5], o[6], o[7]);
+    }
+}
+
+// per-workgroup min dt / max |R| partial, combined later by k_reduce_stage (device-scope
+// atomics from every workgroup on one address serialise across the XCDs)
+DEV void blockPartial(double dtCand, double rCand, double* partial, uint32_t slot)
+{
+    __shared__ double sMin[BLK / 64], sMax_[BLK / 64];
+    dtCand = warpMin(dtCand);
+    rCand = warpMax(rCand);
+    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+    if (l == 0) { sMin[w] = dtCand; sMax_[w] = rCand; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a0 = sMin[0], b0 = sMax_[0];
+#pragma unroll
+        for (int k = 1; k < BLK / 64; k++) { a0 = fmin(a0, sMin[k]); b0 = fmax(b0, sMax_[k]); }
+        partial[2 * slot] = a0;
+        partial[2 * slot + 1] = b0;
+    }
+}
+// Workgroup barrier for data shared through LDS: waits for this wave's LDS
+// operations only.  __syncthreads() (and an LDS-scope fence, which covers the
+// direct global-to-LDS copies) also waits for every outstanding global access,
+// which would stall on the next tile's prefetch.  The "memory" clobber keeps the
+// compiler from moving memory accesses across it.
+DEV void ldsBarrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// newDt = min over the stage's workgroup partials; Rmax = max with the step's running value
+void launchReduceStage(const double* partial, uint32_t n, DevScalars* sc, int checkActive, hipStream_t st);
+
+}  // namespace ebb
