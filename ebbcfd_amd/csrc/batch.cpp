@@ -4,8 +4,8 @@
 // the first mesh (source/integrators.d:56-75).  Here each admitted solve is an ordinary
 // solver (its state, geometry and scratch resident in HBM), and a time-loop step for all of
 // them is one launch per kernel: per RK stage the gradient kernel over every mesh's cell
-// blocks and the face/update kernel over every mesh's face tiles, then one RMS kernel and
-// one epilogue for all meshes.  Every workgroup runs the solo kernels' code on one
+// blocks and the face/update kernel over every mesh's face tiles; each step's epilogue rides in
+// the next step's first gradient launch.  Every workgroup runs the solo kernels' code on one
 // (mesh, block/tile) item, so each mesh's states and history equal its solo run's bit
 // for bit.  The step sequence is captured once as a HIP graph of `graphSteps` steps and
 // replayed; meshes that stop (tEnd, maxSteps, the rho-RMS drop of extensions.rmsDrop, an
@@ -42,8 +42,8 @@ struct BatchGroup {
     int nst = 0;
     int limit[4] = {0, 0, 0, 0};
     uint32_t lds = 0;
-    std::vector<uint2> grad, tile;
-    DBuf<uint2> dGrad, dTile;
+    std::vector<uint2> grad, tile, epi;
+    DBuf<uint2> dGrad, dTile, dEpi;
 };
 
 using GroupKey = std::tuple<int, int, int, int, int, int, int, int, int, int, int, int, int>;
@@ -78,10 +78,11 @@ struct ebb_batch {
     std::vector<uint32_t> slotOf;                 // running member index of each slot
     std::vector<MemberArgs> hmem;
     DBuf<MemberArgs> dmem;
-    std::vector<uint2> rms;
-    DBuf<uint2> dRms;
-    std::vector<uint32_t> fin, force;
-    DBuf<uint32_t> dFin, dForce;
+    std::vector<uint2> epi;                       // every group's epilogue items
+    DBuf<uint2> dEpi;
+    bool ride = true;                             // epilogues ride in the next step's gradient launches
+    std::vector<uint32_t> fin;
+    DBuf<uint32_t> dFin;
     DBuf<DevScalars> dScal;
     DevScalars* hScal = nullptr;
     size_t hScalCap = 0;
@@ -131,9 +132,6 @@ MemberArgs memberArgs(ebb_solver* s)
     }
     s->cur = saved;
     M.parityFlip = uint32_t(saved);
-    M.f = forceArgs(s);
-    const uint64_t nb = uint64_t(s->b.nCells) / 16;
-    M.nRmsFull = uint32_t(nb / RMS_CHUNK_BLOCKS);
     return M;
 }
 
@@ -166,12 +164,14 @@ int rebuild(ebb_batch* b)
 {
     dropGraph(b);
     { int rc = followSpread(b); if (rc) return rc; }
+    for (auto& g : b->groups) { g.dGrad.release(); g.dTile.release(); g.dEpi.release(); }
     b->groups.clear();
     b->hmem.clear();
     b->slotOf.clear();
-    b->rms.clear();
+    b->epi.clear();
     b->fin.clear();
-    b->force.clear();
+    b->ride = true;
+    for (auto& mb : b->members) if (mb.running && !mb.s->rideEpilogue) b->ride = false;
     b->maxStages = 0;
     std::map<GroupKey, size_t> gidx;
     for (size_t k = 0; k < b->members.size(); k++) {
@@ -196,27 +196,26 @@ int rebuild(ebb_batch* b)
         BatchGroup& g = b->groups[it->second];
         b->maxStages = std::max(b->maxStages, g.nst);
         g.lds = std::max(g.lds, s->ftiles.ldsBytes);
-        if (deferForce(s)) {
-            g.grad.push_back(make_uint2(slot, FORCE_ITEM));
-            b->force.push_back(slot);
+        for (uint32_t x = 0; x < b->hmem.back().d[0].nEpi; x++) {
+            g.epi.push_back(make_uint2(slot, x));
+            b->epi.push_back(make_uint2(slot, x));
         }
         // gradient items: cell blocks, or on gradient tiles the border blocks (at least one,
         // whose block 0 resets the step's Rmax)
         const uint32_t nblk = s->useGradTiles ? std::max<uint32_t>(1u, (s->ftiles.nBorder + 255) / 256) : (s->N + 255) / 256;
         for (uint32_t x = 0; x < nblk; x++) g.grad.push_back(make_uint2(slot, x));
         for (uint32_t x = 0; x < s->ftiles.nTiles; x++) g.tile.push_back(make_uint2(slot, x));
-        for (uint32_t x = 0; x < b->hmem.back().nRmsFull + 3; x++) b->rms.push_back(make_uint2(slot, x));
         b->fin.push_back(slot);
     }
     HIPCHK(hipSetDevice(b->device));
     for (auto& g : b->groups) {
         HIPCHK(uploadVec(g.dGrad, g.grad));
         HIPCHK(uploadVec(g.dTile, g.tile));
+        HIPCHK(uploadVec(g.dEpi, g.epi));
     }
     HIPCHK(uploadVec(b->dmem, b->hmem));
-    HIPCHK(uploadVec(b->dRms, b->rms));
+    HIPCHK(uploadVec(b->dEpi, b->epi));
     HIPCHK(uploadVec(b->dFin, b->fin));
-    HIPCHK(uploadVec(b->dForce, b->force));
     if (b->hScalCap < b->fin.size()) {
         if (b->hScal) (void)hipHostFree(b->hScal);
         b->hScal = nullptr;
@@ -229,28 +228,30 @@ int rebuild(ebb_batch* b)
     return EBB_OK;
 }
 
-// one time-loop step of every running member: parity 0 reads each member's current state
-void launchStep(ebb_batch* b, uint32_t parity)
+// one time-loop step of every running member: parity 0 reads each member's current state.
+// afterStep: the step before it in the same sequence has left its epilogue to this one's first
+// gradient launches; lastStep: no step follows in the sequence.
+void launchStep(ebb_batch* b, uint32_t parity, bool afterStep, bool lastStep)
 {
     for (int st = 0; st < b->maxStages; st++) {
         for (auto& g : b->groups)
             if (st < g.nst)
                 launchGradientBatch(g.shape, g.limit[st], b->dmem.p, g.dGrad.p, uint32_t(g.grad.size()), parity,
-                                    uint32_t(st), b->stream);
+                                    uint32_t(st), g.dEpi.p, st == 0 && afterStep && b->ride ? uint32_t(g.epi.size()) : 0u,
+                                    b->stream);
         for (auto& g : b->groups)
             if (st < g.nst)
                 launchFaceTilesBatch(g.shape, g.limit[st], b->dmem.p, g.dTile.p, uint32_t(g.tile.size()), g.lds,
                                      parity, uint32_t(st), b->stream);
     }
-    launchRmsBatch(b->dmem.p, b->dRms.p, uint32_t(b->rms.size()), parity, b->stream);
-    launchFinalizeBatch(b->dmem.p, b->dFin.p, uint32_t(b->fin.size()), parity, b->stream);
+    if (lastStep || !b->ride) launchEpilogueBatch(b->dmem.p, b->dEpi.p, uint32_t(b->epi.size()), parity, b->stream);
 }
 
 int captureGraph(ebb_batch* b)
 {
     dropGraph(b);
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < b->graphSteps; k++) launchStep(b, uint32_t(k & 1));
+    for (int k = 0; k < b->graphSteps; k++) launchStep(b, uint32_t(k & 1), k > 0, k + 1 == b->graphSteps);
     HIPCHK(hipStreamEndCapture(b->stream, &b->graph));
     HIPCHK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     return EBB_OK;
@@ -288,8 +289,8 @@ int runSteps(ebb_batch* b, int64_t steps)
         if (!b->exec) { int rc = captureGraph(b); if (rc) return rc; }
         for (; done + G <= steps; done += G) HIPCHK(hipGraphLaunch(b->exec, b->stream));
     }
-    for (; done < steps; done++) launchStep(b, uint32_t(done & 1));
-    launchPendingForceBatch(b->dmem.p, b->dForce.p, uint32_t(b->force.size()), b->stream);
+    for (const int64_t first = done; done < steps; done++)
+        launchStep(b, uint32_t(done & 1), done > first, done + 1 == steps);
     launchGatherScalars(b->dmem.p, b->dFin.p, uint32_t(n), b->dScal.p, b->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(b->hScal, b->dScal.p, n * sizeof(DevScalars), hipMemcpyDeviceToHost, b->stream));
@@ -626,8 +627,8 @@ void ebb_batch_destroy(ebb_batch* b)
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     dropGraph(b);
     for (auto& mb : b->members) ebb_solver_destroy(mb.s);
-    for (auto& g : b->groups) { g.dGrad.release(); g.dTile.release(); }
-    b->dmem.release(); b->dRms.release(); b->dFin.release(); b->dForce.release(); b->dScal.release();
+    for (auto& g : b->groups) { g.dGrad.release(); g.dTile.release(); g.dEpi.release(); }
+    b->dmem.release(); b->dEpi.release(); b->dFin.release(); b->dScal.release();
     if (b->hScal) (void)hipHostFree(b->hScal);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;

@@ -39,29 +39,17 @@ struct DevScalars {
     int64_t incIters;               // cflAdjust counter
     int64_t steps;                  // completed steps
     int32_t active;                 // 0 once t >= tEnd, maxSteps, convergence or an error was recorded
+    int32_t specActive;             // what the first gradient kernel of a step goes by: `active` as the step
+                                    // before it left it may still be on its way (StageArgs::spec)
     int32_t converged;              // 1 once the rho RMS dropped by rmsDrop below its first-step value
+    uint32_t ticket;                // epilogue workgroups of the current step that are done
     double rms[4];
     double force[2];
     double fsum[2];                 // boundary force sums of the current step, before the AoA rotation
-    int32_t forcePending;           // 1: the last step's boundary force is still to be summed
-    int32_t pad2;
-    int64_t forceSlot;              // its history row (index into the history buffer), -1: none
+    double stageSum[2];             // its newDt and Rmax, on their way to the epilogue's last workgroup
     unsigned long long errBC;       // (stage << 32) | boundary face whose total-conditions inflow has no
                                     // non-negative Mach root (solve.d:648-671), min wins; ~0 = none
     double rms0;                    // rho RMS residual of the first step (convergence stop)
-};
-
-// The ordered boundary-force sum of a time-loop step (mesh.d:645-671), when it is
-// left to the next gradient kernel: one extra workgroup of that kernel sums it while
-// the others compute gradients, so its long dependent chain of additions is off the
-// step's critical path.  The face fluxes it reads are only rewritten by the tile
-// kernel that follows.
-struct ForceArgs {
-    const uint32_t* faces;   // force-boundary faces in bGroups order
-    uint32_t n;              // 0: no force boundary (no extra workgroup)
-    const double* lenF;      // len*flux per face
-    double rot[4];           // freestream AoA rotation (row-major)
-    double* hist;            // history rows (HIST_FIELDS doubles each)
 };
 
 struct DevMesh {
@@ -137,13 +125,17 @@ struct StageArgs {
     int first;             // first stage of a step (resets Rmax)
     int last;              // last stage of a step (NaN scan of the new state)
     int checkActive;       // honour sc->active (time loop) or always run
-    int deferReduce;       // leave the partials for the step's RMS kernel instead of reducing them now
+    int deferReduce;       // leave the partials for the step's epilogue instead of reducing them now
     int recordErrors;
     uint32_t stageId;      // global stage counter for error ordering
     uint32_t stepId;
     int order;             // bit 0: the face/update tile kernel walks each XCD's slice of tiles
                            // last to first; bit 1: the gradient kernel its slice of cell blocks
-    ForceArgs force;       // gradient kernels: the pending boundary force, if any
+    int spec;              // first stage of a time-loop step whose gradient kernel also carries the epilogue
+                           // of the step before: that kernel runs as long as the step before ran, and the
+                           // tile (or face) kernel after it passes on whether the loop goes on
+    double4* ghostSave;    // spec: receives the ghost rows the gradient kernel replaces, so that a loop that
+                           // turns out to have ended gets them back
 };
 
 // Tiles for the fused stage kernel: each tile is a compact group of interior
@@ -240,17 +232,21 @@ struct FaceTileArgs {
     uint32_t pad;
 };
 
+struct DiagArgs;
+
 // Launchers (kernels.hip).  All run on `stream`.
 void launchFaceTiles(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, int S,
                      hipStream_t stream);
 void launchStageTiles(const DevMesh& m, const PhysParams& p, const StageArgs& a, const TileArgs& t, int S,
                       hipStream_t stream);
-// gradient tiles: the border kernel (ring cells' gradients; the force and Rmax duties of the
+// gradient tiles: the border kernel (ring cells' gradients; the epilogue and Rmax duties of the
 // gradient kernel) then the tile kernel (own gradients, faces and update); parts 1: the border
 // kernel only, 2: the tile kernel (and the stage reduction) only
 void launchGradTiles(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, int S,
-                     hipStream_t stream, int parts = 3);
-void launchGradient(const DevMesh& m, const PhysParams& p, const StageArgs& a, int S, hipStream_t stream);
+                     hipStream_t stream, int parts = 3, const DiagArgs* epi = nullptr);
+// epi: the epilogue of the step before, carried as extra workgroups (null: none)
+void launchGradient(const DevMesh& m, const PhysParams& p, const StageArgs& a, int S, hipStream_t stream,
+                    const DiagArgs* epi = nullptr);
 void launchFaces(const DevMesh& m, const PhysParams& p, const StageArgs& a, hipStream_t stream);
 void launchUpdate(const DevMesh& m, const PhysParams& p, const StageArgs& a, int S, hipStream_t stream);
 
@@ -259,9 +255,8 @@ struct DiagArgs {
     const double4* qold;     // state before the step
     uint32_t N, L;           // interior cells, cells incl. ghosts (reference array length)
     const uint32_t* perm;    // reference index -> device index (null = identity)
-    const double* blockSums; // per 16-element block, its 8 leaf sums from the last stage (null: read the states)
-    double* chunkTrees;      // nChunks * 8 * 16 partial pairwise trees
-    uint32_t* chunkMask;     // nChunks * 8 bit masks of the levels present
+    const double* blockSums; // per 16-element block of the L cells, its 8 leaf sums (zero past the interior)
+    double* chunkTops;       // per full chunk of RMS_CHUNK_BLOCKS blocks, its 8 sums; then the fold of the rest
     const uint32_t* forceFaces; uint32_t nForce;
     const double* lenF;
     double rot[4];           // freestream AoA rotation (row-major)
@@ -271,11 +266,11 @@ struct DiagArgs {
     int64_t histBase;        // step index of hist[0]
     int64_t histCap;
     int64_t maxSteps;        // stop after this many completed steps (<0: none)
-    // stage partials left by the step's stages (deferReduce): stage s holds nPart
-    // (min dt candidate, max |R|) pairs at partial + s * pstride; nStages 0: none
+    // stage partials left by the step's stages (deferReduce): nPart (min dt candidate, max |R|)
+    // pairs per stage, stage after stage
     const double* partial;
-    uint32_t nPart, pstride, nStages;
-    int deferForce;          // 1: the force is left pending for the next gradient kernel
+    uint32_t nPart, nStages;
+    uint32_t nEpi;           // workgroups of the epilogue (epilogueBody)
     int histRing;            // 1: history row = steps % histCap (batched runs) instead of steps - histBase
     double rmsDrop;          // > 0: stop once rho RMS <= rmsDrop * its first-step value
     DevScalars* sc;
@@ -285,46 +280,44 @@ constexpr int HIST_RING_ROWS = 256;   // rows of a solver's device history ring
 
 // Batched runs (many meshes per launch): the per-mesh arguments of every kernel of a
 // time-loop step, kept in device memory, one record per mesh.  A work item (mesh, local
-// index) names a cell block of the gradient kernel (FORCE_ITEM: that mesh's pending
-// boundary force), a face tile, or a workgroup of the RMS kernel; each workgroup runs the
-// solo kernels' code on its item, so every mesh's results equal its solo run's.
+// index) names a cell block of the gradient kernel, a face tile, or a workgroup of the step
+// epilogue; each workgroup runs the solo kernels' code on its item, so every mesh's results
+// equal its solo run's.
 struct MemberArgs {
     DevMesh m;
     PhysParams p;
     FaceTileArgs t;
     StageArgs st[2][4];      // [parity][stage in step]: parity 0 reads the state buffer qA
-    DiagArgs d[2];           // [parity] the step's RMS kernel and epilogue
-    ForceArgs f;             // the pending boundary force at the end of a run
+    DiagArgs d[2];           // [parity] the step's epilogue
     uint32_t parityFlip;     // 1: the mesh's current state is in qB (its parity is the batch's ^ 1)
-    uint32_t nRmsFull;       // full RMS chunks (k_rms_blocks' nfull)
-    uint32_t pad[2];
+    uint32_t pad[3];
 };
-constexpr uint32_t FORCE_ITEM = 0xFFFFFFFFu;
-constexpr uint32_t RMS_CHUNK_BLOCKS = 1024;     // 16-element blocks per workgroup
-void launchRmsChunks(const DiagArgs& d, hipStream_t stream);
-// sums a pending boundary force (end of a time-loop batch); no-op when none is pending
-void launchPendingForce(const ForceArgs& f, DevScalars* sc, hipStream_t stream);
-void launchFinalize(const DiagArgs& d, hipStream_t stream);
+constexpr uint32_t RMS_CHUNK_BLOCKS = 1024;     // 16-element blocks per epilogue workgroup
+void launchRmsLeaves(const DiagArgs& d, double* blockSums, hipStream_t stream);
+// the epilogue of a step as a launch of its own
+void launchEpilogue(const DiagArgs& d, hipStream_t stream);
 void launchInitScalars(DevScalars* sc, double dt, double t, double CFL, hipStream_t stream);
 
 // Batched launches over many meshes (one launch per kernel for all of them).  The kernel
 // shape (S, flux, viscous, order, limiter mode, precision) is the group's; items are
-// (mesh record, local index).  parity selects each mesh's state buffers (see MemberArgs).
+// (mesh record, local index).  epi: the epilogue items of the step before, at parity ^ 1, that
+// a first gradient launch carries.  parity selects each mesh's state buffers (see MemberArgs).
 struct GroupShape {
     int S, flux, viscous, order, limited, venkat, mixed;
     int gradTiles;   // 1: gradient items are border blocks and tiles compute their own gradients
 };
 void launchGradientBatch(const GroupShape& g, int limitStage, const MemberArgs* mem, const uint2* items,
-                         uint32_t nItems, uint32_t parity, uint32_t stage, hipStream_t stream);
+                         uint32_t nItems, uint32_t parity, uint32_t stage, const uint2* epi, uint32_t nEpi,
+                         hipStream_t stream);
 void launchFaceTilesBatch(const GroupShape& g, int limitStage, const MemberArgs* mem, const uint2* items,
                           uint32_t nItems, uint32_t ldsBytes, uint32_t parity, uint32_t stage, hipStream_t stream);
-void launchRmsBatch(const MemberArgs* mem, const uint2* items, uint32_t nItems, uint32_t parity, hipStream_t stream);
-void launchFinalizeBatch(const MemberArgs* mem, const uint32_t* members, uint32_t n, uint32_t parity,
-                         hipStream_t stream);
-void launchPendingForceBatch(const MemberArgs* mem, const uint32_t* members, uint32_t n, hipStream_t stream);
+// the epilogue items (mesh, workgroup) of a step run at `parity`
+void launchEpilogueBatch(const MemberArgs* mem, const uint2* epi, uint32_t nEpi, uint32_t parity, hipStream_t stream);
 // copies each listed mesh's DevScalars into out[k] (one host copy for all)
 void launchGatherScalars(const MemberArgs* mem, const uint32_t* members, uint32_t n, DevScalars* out,
                          hipStream_t stream);
+// ghost rows q[0..n) back from `save`, and their FP32 shadow (null on the FP64 path)
+void launchRestoreGhosts(double4* q, float4* q32, const double4* save, uint32_t n, hipStream_t stream);
 // FP32 shadow q32[0..n) of q[0..n) (mixed precision)
 void launchShadow(const double4* q, float4* q32, uint32_t n, hipStream_t stream);
 

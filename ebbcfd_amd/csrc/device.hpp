@@ -15,7 +15,6 @@ namespace ebb {
 constexpr double G_ = 1.4;
 constexpr int BLK = 256;
 static_assert(uint32_t(BLK) == FACE_TILE_LANES, "face tile padding assumes one lane per workgroup thread");
-constexpr int FORCE_LDS = 1024;   // force faces staged per pass by a gradient kernel's force workgroup
 
 enum { BT_FULL = 0, BT_CONSTP, BT_INVWALL, BT_VISCWALL, BT_SYM, BT_TPIN, BT_DIRICHLET };
 
@@ -514,74 +513,6 @@ DEV bool ghostFromOwner(const BFace& bf, const double qo[4], const double4* qbuf
     return ghostState(bf, qo, qg, old);
 }
 
-// The boundary force sum of mesh.d:645-671: (len*flux) momentum components of the
-// force faces added in order, two interleaved chains, by thread 0 (its result).
-// fp: LDS staging of CAP (x, y) pairs.
-template <int NT, int CAP>
-DEV void orderedForce(const uint32_t* faces, uint32_t nF, const double* lenF, double2* fp, double& f0, double& f1)
-{
-    f0 = 0; f1 = 0;
-    for (uint32_t k0 = 0; k0 < nF; k0 += CAP) {
-        const uint32_t cnt = (nF - k0) < uint32_t(CAP) ? (nF - k0) : uint32_t(CAP);
-        __syncthreads();
-        // all of a thread's face ids, then all of their fluxes, are loaded before any is
-        // used: two round trips per pass instead of two per face
-        constexpr int FS = (CAP + NT - 1) / NT;
-        uint32_t fi[FS];
-#pragma unroll
-        for (int u = 0; u < FS; u++) {
-            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
-            fi[u] = x < cnt ? faces[k0 + x] : 0u;
-        }
-        double2 fv[FS];
-#pragma unroll
-        for (int u = 0; u < FS; u++) {
-            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
-            fv[u] = x < cnt ? make_double2(lenF[size_t(fi[u]) * 4 + 1], lenF[size_t(fi[u]) * 4 + 2])
-                            : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < FS; u++) {
-            const uint32_t x = threadIdx.x + uint32_t(u) * NT;
-            if (x < cnt) fp[x] = fv[u];
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            // the two ordered chains interleave; 32 LDS reads are in flight ahead of the adds
-            uint32_t x = 0;
-            for (; x + 32 <= cnt; x += 32) {
-                double2 v[32];
-#pragma unroll
-                for (int u = 0; u < 32; u++) v[u] = fp[x + u];
-#pragma unroll
-                for (int u = 0; u < 32; u++) { f0 += v[u].x; f1 += v[u].y; }
-            }
-            for (; x < cnt; x++) { const double2 v = fp[x]; f0 += v.x; f1 += v.y; }
-        }
-    }
-}
-
-// a pending force (k_finalize left it): rotated drag/lift into the step's history row
-// and the scalars, as k_finalize would have written them
-template <int NT, int CAP>
-DEV void pendingForce(const ForceArgs& f, DevScalars* sc, double2* fp)
-{
-    if (!sc->forcePending) return;
-    double f0, f1;
-    orderedForce<NT, CAP>(f.faces, f.n, f.lenF, fp, f0, f1);
-    if (threadIdx.x == 0) {
-        const double ld0 = 0.0 + f.rot[0] * f0 + f.rot[1] * f1;
-        const double ld1 = 0.0 + f.rot[2] * f0 + f.rot[3] * f1;
-        const int64_t slot = sc->forceSlot;
-        if (slot >= 0) {
-            double* h = f.hist + slot * HIST_FIELDS;
-            h[7] = ld0; h[8] = ld1;
-        }
-        sc->force[0] = ld0; sc->force[1] = ld1;
-        sc->forcePending = 0;
-    }
-}
-
 // MODE 0: ghost states only (order 1); 1: unlimited gradient (no limiter stored);
 // 2: scalar limiter; 3: scalar limiter followed by the LP vector limiter (lim
 // stored as x,y pairs).
@@ -590,8 +521,7 @@ DEV void pendingForce(const ForceArgs& f, DevScalars* sc, double2* fp)
 // centroid offsets in FP64, converted); gradients and limiters are stored as FP32
 // rows (32 + 16 bytes per cell); each ghost is written to the shadow and, widened, to
 // the FP64 row.
-// LDS of one gradient workgroup: staging of the gradient rows (and of the force faces)
-// and of the limiter rows
+// LDS of one gradient workgroup: staging of the gradient rows and of the limiter rows
 template <int MODE>
 struct GradLds {
     static constexpr int LWS = MODE == 3 ? 8 : ((MODE == 2 || MODE == 4) ? 4 : 0);
@@ -647,6 +577,8 @@ DEV void cellGradient(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     for (int j = 0; j < S; j++)
         if (nb[j] >= m.N) {
             const BFace& bf = m.bface[nb[j] - m.N];
+            if (storeGhosts && a.ghostSave)
+                a.ghostSave[nb[j] - m.N] = make_double4(qn[j][0], qn[j][1], qn[j][2], qn[j][3]);
             R old[4] = {0, 0, 0, 0};
             if (bf.type == BT_TPIN) {
 #pragma unroll
@@ -667,6 +599,21 @@ DEV void cellGradient(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     gradLimit<S, MODE, R>(qi, qn, nullptr, 0, ci, cn, real, a.limit, p.lpThresh, g, lx, ly, eps2);
 }
 
+// whether a stage's gradient kernel runs
+DEV bool stageRuns(const StageArgs& a)
+{
+    return !a.checkActive || (a.spec ? a.sc->specActive : a.sc->active);
+}
+
+// whether the tile or face kernel of a stage runs; one thread of a step's first one passes a loop
+// that has ended on to the next step's gradient kernel
+DEV bool fluxRuns(const StageArgs& a, bool first)
+{
+    if (!a.checkActive || a.sc->active) return true;
+    if (first && a.spec) a.sc->specActive = 0;
+    return false;
+}
+
 // One workgroup of the gradient kernel on cell block `bid` of its mesh (the solo and the
 // batched kernels run this same code).
 template <int S, int MODE, int MIX>
@@ -676,8 +623,9 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     constexpr int LWS = GradLds<MODE>::LWS;
     auto& sg = L.sg;
     auto& sl = L.sl;
-    if (a.checkActive && !a.sc->active) return;
-    if (bid == 0 && threadIdx.x == 0 && a.first) a.sc->rmaxBits = 0;   // Rmax is per step
+    if (!stageRuns(a)) return;
+    // Rmax is per step (the time loop's epilogue takes it from the stages' partials instead)
+    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;
     const uint32_t i = bid * BLK + threadIdx.x;
     if (MODE == 0 && i >= m.N) return;
     const bool have = i < m.N;   // no early return below: the staged stores need every thread
@@ -693,7 +641,8 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
                 if (nb >= m.N) {
                     const BFace& bf = m.bface[nb - m.N];
                     R qg[4], old[4] = {0, 0, 0, 0};
-                    if (bf.type == BT_TPIN) ldStage<MIX>(a, nb, old);
+                    if (bf.type == BT_TPIN || a.ghostSave) ldStage<MIX>(a, nb, old);
+                    if (a.ghostSave) a.ghostSave[nb - m.N] = make_double4(old[0], old[1], old[2], old[3]);
                     if (!ghostState<R>(bf, qi, qg, old) && a.recordErrors)
                         atomicMin(&a.sc->errBC, (uint64_t(a.stageId) << 32) | (nb - m.N));
                     stGhostRow<MIX>(a, nb, qg);

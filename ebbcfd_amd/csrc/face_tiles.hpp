@@ -181,7 +181,7 @@ DEV void faceTileBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     uint4 rNext = t.fref[size_t(tile) * t.faceStride + tid];
     const uint4 d = t.desc[tile];
     // the loop's active flag is read after those loads are issued (all in bounds)
-    if (a.checkActive && !a.sc->active) return;
+    if (!fluxRuns(a, pslot == 0 && tid == 0)) return;
     const uint32_t nF = d.y;
     for (uint32_t k = tid; k < nF; k += BLK) {
         const uint4 r = rNext;   // cell a, cell b, node 0, node 1

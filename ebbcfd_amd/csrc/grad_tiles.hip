@@ -1,5 +1,6 @@
 // The gradient-tile stage kernels (extensions.stagePath = "gradTiles") for cells of STRIDE slots
 // (compiled once per stride).
+#include "epilogue.hpp"
 #include "face_tiles.hpp"
 #include "tile_launch.hpp"
 
@@ -27,8 +28,8 @@ template <int S, int MODE, int MIX>
 DEV void borderGradBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, uint32_t bid)
 {
     using R = RealOf<MIX>;
-    if (a.checkActive && !a.sc->active) return;
-    if (bid == 0 && threadIdx.x == 0 && a.first) a.sc->rmaxBits = 0;   // Rmax is per step
+    if (!stageRuns(a)) return;
+    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;   // Rmax is per step
     const uint32_t k = bid * BLK + threadIdx.x;
     if (k >= t.nBorder) return;
     const uint32_t i = t.border[k];
@@ -47,18 +48,19 @@ DEV void borderGradBody(const DevMesh& m, const PhysParams& p, const StageArgs& 
     }
 }
 
-// Workgroup 0 sums a pending boundary force when there is one (as the gradient kernel's
-// force workgroup); the others are border blocks.
+// The first epiPad workgroups carry the epilogue of the step before (as the gradient kernel's);
+// the others are border blocks.
 template <int S, int MODE, int MIX>
-__global__ __launch_bounds__(BLK) void k_border_grad(DevMesh m, PhysParams p, StageArgs a, FaceTileArgs t)
+__global__ __launch_bounds__(BLK) void k_border_grad(DevMesh m, PhysParams p, StageArgs a, FaceTileArgs t, DiagArgs d,
+                                                     uint32_t epiPad)
 {
-    __shared__ double2 fstage[FORCE_LDS];
-    const uint32_t fw = a.force.n ? 1u : 0u;
-    if (fw && blockIdx.x == 0) {
-        pendingForce<BLK, FORCE_LDS>(a.force, a.sc, fstage);
+    if (blockIdx.x < epiPad) {
+        __shared__ double staging[2 * FORCE_LDS];
+        __shared__ EpiLds E;
+        if (blockIdx.x < d.nEpi) epilogueBody(d, blockIdx.x, E, staging);
         return;
     }
-    borderGradBody<S, MODE, MIX>(m, p, a, t, xcdBlock(blockIdx.x - fw, gridDim.x - fw));
+    borderGradBody<S, MODE, MIX>(m, p, a, t, xcdBlock(blockIdx.x - epiPad, gridDim.x - epiPad));
 }
 
 // One workgroup of the gradient-tile kernel on tile `tile`.  MODE 1: an unlimited stage
@@ -77,7 +79,7 @@ DEV void gradTileBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     uint32_t sNext = t.fslot[size_t(tile) * t.faceStride + tid];
     const uint4 d = t.desc[tile];
     const uint32_t nH = t.nHalo[tile];
-    if (a.checkActive && !a.sc->active) return;
+    if (!fluxRuns(a, pslot == 0 && tid == 0)) return;
     const uint32_t nC = d.x, nF = d.y;
     R* gl = reinterpret_cast<R*>(lds);
     const FaceLds<MIX> fl(lds + t.glDoubles, t.faceStride + 1);
@@ -178,23 +180,25 @@ __global__ __launch_bounds__(BLK, 3) void k_grad_tile(DevMesh m, PhysParams p, S
 
 template <int S, int FLUX, int VISC, int MIX>
 static void gradTileM(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, int mode,
-                      int parts, hipStream_t st)
+                      int parts, const DiagArgs* epi, hipStream_t st)
 {
     const dim3 g(t.nTiles), b(BLK);
     const uint32_t nb = (t.nBorder + BLK - 1) / BLK;
-    const dim3 gb((nb ? nb : 1u) + (a.force.n ? 1u : 0u));   // at least one workgroup: the Rmax reset
+    const DiagArgs d = epi ? *epi : DiagArgs{};
+    const uint32_t pad = epiPadding(d.nEpi);
+    const dim3 gb((nb ? nb : 1u) + pad);   // at least one workgroup: the Rmax reset
     const bool border = parts & 1, tiles = parts & 2;
     switch (mode) {
     case 1:
-        if (border) hipLaunchKernelGGL((k_border_grad<S, 1, MIX>), gb, b, 0, st, m, p, a, t);
+        if (border) hipLaunchKernelGGL((k_border_grad<S, 1, MIX>), gb, b, 0, st, m, p, a, t, d, pad);
         if (tiles) hipLaunchKernelGGL((k_grad_tile<S, FLUX, VISC, 1, MIX>), g, b, t.ldsBytes, st, m, p, a, t);
         break;
     case 4:
-        if (border) hipLaunchKernelGGL((k_border_grad<S, 4, MIX>), gb, b, 0, st, m, p, a, t);
+        if (border) hipLaunchKernelGGL((k_border_grad<S, 4, MIX>), gb, b, 0, st, m, p, a, t, d, pad);
         if (tiles) hipLaunchKernelGGL((k_grad_tile<S, FLUX, VISC, 4, MIX>), g, b, t.ldsBytes, st, m, p, a, t);
         break;
     default:
-        if (border) hipLaunchKernelGGL((k_border_grad<S, 2, MIX>), gb, b, 0, st, m, p, a, t);
+        if (border) hipLaunchKernelGGL((k_border_grad<S, 2, MIX>), gb, b, 0, st, m, p, a, t, d, pad);
         if (tiles) hipLaunchKernelGGL((k_grad_tile<S, FLUX, VISC, 2, MIX>), g, b, t.ldsBytes, st, m, p, a, t);
         break;
     }
@@ -202,12 +206,12 @@ static void gradTileM(const DevMesh& m, const PhysParams& p, const StageArgs& a,
 
 template <int S>
 void gradTileS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, int mode,
-                      int parts, hipStream_t st)
+                      int parts, const DiagArgs* epi, hipStream_t st)
 {
 #define EBB_GT(F, V)                                                      \
     do {                                                                  \
-        if (p.mixed) gradTileM<S, F, V, 1>(m, p, a, t, mode, parts, st);  \
-        else gradTileM<S, F, V, 0>(m, p, a, t, mode, parts, st);          \
+        if (p.mixed) gradTileM<S, F, V, 1>(m, p, a, t, mode, parts, epi, st);  \
+        else gradTileM<S, F, V, 0>(m, p, a, t, mode, parts, epi, st);          \
     } while (0)
     if (p.flux == 1) {
         if (p.viscous) EBB_GT(1, 1); else EBB_GT(1, 0);
@@ -219,17 +223,21 @@ void gradTileS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const 
 
 template <int S, int MODE, int MIX>
 __global__ __launch_bounds__(BLK) void k_border_grad_batch(const MemberArgs* __restrict__ mem,
-                                                           const uint2* __restrict__ items, uint32_t parity, uint32_t stage)
+                                                           const uint2* __restrict__ items, uint32_t parity, uint32_t stage,
+                                                           const uint2* __restrict__ epi, uint32_t nEpi, uint32_t epiPad)
 {
-    __shared__ double2 fstage[FORCE_LDS];
-    const uint2 it = items[xcdBlock(blockIdx.x, gridDim.x)];
-    const MemberArgs& M = mem[it.x];
-    const StageArgs& a = M.st[parity ^ M.parityFlip][stage];
-    if (it.y == FORCE_ITEM) {
-        pendingForce<BLK, FORCE_LDS>(a.force, a.sc, fstage);
+    if (blockIdx.x < epiPad) {
+        __shared__ double staging[2 * FORCE_LDS];
+        __shared__ EpiLds E;
+        if (blockIdx.x >= nEpi) return;
+        const uint2 it = epi[blockIdx.x];
+        const DiagArgs d = mem[it.x].d[parity ^ 1u ^ mem[it.x].parityFlip];   // scalar loads, before any store
+        epilogueBody(d, it.y, E, staging);
         return;
     }
-    borderGradBody<S, MODE, MIX>(M.m, M.p, a, M.t, it.y);
+    const uint2 it = items[xcdBlock(blockIdx.x - epiPad, gridDim.x - epiPad)];
+    const MemberArgs& M = mem[it.x];
+    borderGradBody<S, MODE, MIX>(M.m, M.p, M.st[parity ^ M.parityFlip][stage], M.t, it.y);
 }
 
 template <int S, int FLUX, int VISC, int MODE, int MIX>
@@ -244,13 +252,14 @@ __global__ __launch_bounds__(BLK, 3) void k_grad_tile_batch(const MemberArgs* __
 
 template <int S, int MIX>
 void borderBatchS(int mode, const MemberArgs* mem, const uint2* items, uint32_t n, uint32_t par, uint32_t st,
-                         hipStream_t s)
+                  const uint2* epi, uint32_t nEpi, hipStream_t s)
 {
-    const dim3 g(n), b(BLK);
+    const uint32_t pad = epiPadding(nEpi);
+    const dim3 g(n + pad), b(BLK);
     switch (mode) {
-    case 1: hipLaunchKernelGGL((k_border_grad_batch<S, 1, MIX>), g, b, 0, s, mem, items, par, st); break;
-    case 4: hipLaunchKernelGGL((k_border_grad_batch<S, 4, MIX>), g, b, 0, s, mem, items, par, st); break;
-    default: hipLaunchKernelGGL((k_border_grad_batch<S, 2, MIX>), g, b, 0, s, mem, items, par, st); break;
+    case 1: hipLaunchKernelGGL((k_border_grad_batch<S, 1, MIX>), g, b, 0, s, mem, items, par, st, epi, nEpi, pad); break;
+    case 4: hipLaunchKernelGGL((k_border_grad_batch<S, 4, MIX>), g, b, 0, s, mem, items, par, st, epi, nEpi, pad); break;
+    default: hipLaunchKernelGGL((k_border_grad_batch<S, 2, MIX>), g, b, 0, s, mem, items, par, st, epi, nEpi, pad); break;
     }
 }
 
@@ -279,9 +288,11 @@ void gradTileBatchS(const GroupShape& gs, int limitStage, const MemberArgs* mem,
 }
 
 template void gradTileS<STRIDE>(const DevMesh&, const PhysParams&, const StageArgs&, const FaceTileArgs&, int, int,
-                                hipStream_t);
-template void borderBatchS<STRIDE, 0>(int, const MemberArgs*, const uint2*, uint32_t, uint32_t, uint32_t, hipStream_t);
-template void borderBatchS<STRIDE, 1>(int, const MemberArgs*, const uint2*, uint32_t, uint32_t, uint32_t, hipStream_t);
+                                const DiagArgs*, hipStream_t);
+template void borderBatchS<STRIDE, 0>(int, const MemberArgs*, const uint2*, uint32_t, uint32_t, uint32_t, const uint2*,
+                                      uint32_t, hipStream_t);
+template void borderBatchS<STRIDE, 1>(int, const MemberArgs*, const uint2*, uint32_t, uint32_t, uint32_t, const uint2*,
+                                      uint32_t, hipStream_t);
 template void gradTileBatchS<STRIDE, 0>(const GroupShape&, int, const MemberArgs*, const uint2*, uint32_t, uint32_t,
                                         uint32_t, uint32_t, hipStream_t);
 template void gradTileBatchS<STRIDE, 1>(const GroupShape&, int, const MemberArgs*, const uint2*, uint32_t, uint32_t,

@@ -100,20 +100,6 @@ void aoaRotation(const ebb_solver* s, double rot[4])
     rot[0] = double(cosl(a)); rot[1] = -double(sinl(a)); rot[2] = double(sinl(a)); rot[3] = double(cosl(a));
 }
 
-// Paths whose stages start with the gradient kernel leave each step's force sum to the
-// next gradient kernel (the fused path sums it in the RMS kernel).
-bool deferForce(const ebb_solver* s) { return !s->useTiles && s->d_forceFaces.n > 0; }
-
-ForceArgs forceArgs(const ebb_solver* s)
-{
-    ForceArgs f{};
-    f.faces = s->d_forceFaces.p; f.n = uint32_t(s->d_forceFaces.n);
-    f.lenF = s->d_lenF.p;
-    aoaRotation(s, f.rot);
-    f.hist = s->d_hist.p;
-    return f;
-}
-
 // The FP32 shadow paired with a state buffer (mixed precision), null otherwise.
 float4* shadowOf(ebb_solver* s, const double4* q)
 {
@@ -161,18 +147,21 @@ StageArgs loopStageArgs(ebb_solver* s, int kind, double4* qin, const double4* qn
     StageArgs a = baseStageArgs(s, kind, qin, qn, qout, limit, dtUpdate, first, last, stageId, stepId);
     a.checkActive = 1;
     a.rmsBlocks = (last && s->rmsFused) ? s->d_rmsBlocks.p : nullptr;
-    // time loop: each stage leaves its partials in its own region; the step's RMS
-    // kernel reduces them (nothing in the step reads newDt or Rmax before that)
+    // time loop: each stage leaves its partials in its own region; the step's epilogue
+    // reduces them (nothing in the step reads newDt or Rmax before that)
     a.deferReduce = 1;
-    a.partial = s->d_partial.p + size_t(stageInStep) * s->pstride;
-    // the gradient kernels of the time loop also sum the previous step's force
-    if (deferForce(s)) a.force = forceArgs(s);
+    a.partial = s->d_partial.p + size_t(stageInStep) * 2 * s->nPart;
+    if (first && s->rideEpilogue) {
+        a.spec = 1;
+        a.ghostSave = s->d_ghostSave.p;   // null on gradient tiles, whose tile kernel stores the ghosts
+    }
     return a;
 }
 
 // one residual evaluation + stage update
 void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qout, int limit, int dtUpdate,
-           int first, int last, int checkActive, double4* R, double4* estate, uint32_t stepId)
+           int first, int last, int checkActive, double4* R, double4* estate, uint32_t stepId,
+           const DiagArgs* epi = nullptr)
 {
     const uint32_t stageId = s->stageCounter++;
     StageArgs a;
@@ -188,18 +177,19 @@ void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qo
     if (s->useTiles && !estate && kind != SK_RESIDUAL) {
         launchStageTiles(s->dm, s->phys, a, s->tiles, int(s->S), s->stream);
     } else if (s->useGradTiles && !estate && kind != SK_RESIDUAL) {
-        launchGradTiles(s->dm, s->phys, a, s->ftiles, int(s->S), s->stream);
+        launchGradTiles(s->dm, s->phys, a, s->ftiles, int(s->S), s->stream, 3, epi);
     } else if (s->useFaceTiles && !estate && kind != SK_RESIDUAL) {
-        launchGradient(s->dm, s->phys, a, int(s->S), s->stream);
+        launchGradient(s->dm, s->phys, a, int(s->S), s->stream, epi);
         launchFaceTiles(s->dm, s->phys, a, s->ftiles, int(s->S), s->stream);
     } else {
-        launchGradient(s->dm, s->phys, a, int(s->S), s->stream);
+        launchGradient(s->dm, s->phys, a, int(s->S), s->stream, epi);
         launchFaces(s->dm, s->phys, a, s->stream);
         launchUpdate(s->dm, s->phys, a, int(s->S), s->stream);
     }
     s->lastInput = qin;
     s->lastLimit = limit;
     s->haveStage = true;
+    s->gradStale = false;
 }
 
 // Integrator.step (source/integrators.d:22-270) from qcur() into qnext(): each stage's
@@ -220,13 +210,16 @@ std::vector<StageDesc> stepSequence(ebb_solver* s)
     }
 }
 
-// Integrator.step: all stages of one step from qcur() into qnext()
-void stepStages(ebb_solver* s, int checkActive, uint32_t stepId)
+// Integrator.step: all stages of one step from qcur() into qnext(); epi: the epilogue of the step
+// before, for the first gradient kernel to carry
+void stepStages(ebb_solver* s, int checkActive, uint32_t stepId, const DiagArgs* epi = nullptr)
 {
     s->stageInStep = 0;
     const double4* q = s->qcur();
-    for (const StageDesc& x : stepSequence(s))
-        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, nullptr, stepId);
+    for (const StageDesc& x : stepSequence(s)) {
+        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, nullptr, stepId, epi);
+        epi = nullptr;
+    }
 }
 
 int stagesPerStep(const Config& c)
@@ -242,8 +235,8 @@ DiagArgs diagArgs(ebb_solver* s, const double4* qnew, const double4* qold, int64
 {
     DiagArgs d{};
     d.qnew = qnew; d.qold = qold; d.N = s->N; d.L = s->N + s->G; d.perm = s->refOf.empty() ? nullptr : s->d_devOf.p;
-    d.blockSums = s->rmsFused ? s->d_rmsBlocks.p : nullptr;
-    d.chunkTrees = s->d_chunkTrees.p; d.chunkMask = s->d_chunkMask.p;
+    d.blockSums = s->d_rmsBlocks.p;
+    d.chunkTops = s->d_chunkTops.p;
     d.forceFaces = s->d_forceFaces.p; d.nForce = uint32_t(s->d_forceFaces.n);
     d.lenF = s->d_lenF.p;
     aoaRotation(s, d.rot);
@@ -251,8 +244,9 @@ DiagArgs diagArgs(ebb_solver* s, const double4* qnew, const double4* qold, int64
     d.dynamicDt = s->cfg.dynamicDt; d.cflAdjust = s->cfg.cflAdjust;
     d.hist = s->d_hist.p; d.histBase = histBase; d.histCap = s->histCap;
     d.maxSteps = maxSteps;
-    d.partial = s->d_partial.p; d.nPart = s->nPart; d.pstride = s->pstride; d.nStages = s->stageInStep;
-    d.deferForce = deferForce(s) ? 1 : 0;
+    d.partial = s->d_partial.p; d.nPart = s->nPart; d.nStages = s->stageInStep;
+    const uint32_t nfull = uint32_t((uint64_t(s->N) + s->G) / 16 / RMS_CHUNK_BLOCKS);
+    d.nEpi = nfull ? nfull + 3 : 1;
     d.histRing = 0;
     d.rmsDrop = s->cfg.rmsDrop;
     d.sc = s->d_sc;
@@ -551,14 +545,13 @@ int64_t estimateDeviceBytes(const BuiltMesh& b, const Config& c)
     bytes += int64_t(1.1 * double(N)) * (4 + 2 * S) + int64_t(1.7 * double(N)) * (16 + 4) + 2 * 256 * 20;
     // gradient tiles: an LDS-row pair per face record, each tile's ring and the border (~0.3 N each)
     if (c.stagePath == 3) bytes += int64_t(1.7 * double(N)) * 4 + int64_t(0.6 * double(N)) * 4 + int64_t(1.1 * double(N)) * 4 * S + 4096;
-    bytes += ((N + 15) / 16) * 64;                         // RMS leaf sums
+    bytes += (C / 16 + 1) * 64;                            // RMS leaf sums
     // tiles: ~700 cells each, or at least two per CU on small meshes (down to 32 cells)
     const int64_t tiles = std::max<int64_t>(N / (c.stagePath == 3 ? 250 : 700) + 1,
                                             c.spreadTiles ? std::min<int64_t>(N / 32 + 1, 512) : 0);
     bytes += (2 * std::max<int64_t>((N + 255) / 256, tiles) + 2) * 4 * 8;   // stage partials
     bytes += 256 * HIST_FIELDS * 8;
-    const int64_t nchunks = (C / 16 + RMS_CHUNK_BLOCKS - 1) / RMS_CHUNK_BLOCKS + 1;
-    bytes += nchunks * (128 * 8 + 32);
+    bytes += (C / 16 / RMS_CHUNK_BLOCKS + 1) * 64 + G * 32;   // chunk tops; ghost rows kept for a loop that ends
     return bytes;
 }
 
@@ -733,16 +726,20 @@ int buildDevice(ebb_solver* s)
     if (!s->refOf.empty()) HIPCHK(trackUpload(s, s->d_devOf, s->devOf));
     // leaf blocks need 16 aligned consecutive reference cells per 16 lanes of the last stage
     s->rmsFused = !s->useTiles && ((s->useFaceTiles || !s->refOf.empty()) ? c.tileOrder == TILE_BLOCKS : true);
-    if (s->rmsFused) HIPCHK((hipError_t)trackAlloc(s, s->d_rmsBlocks, size_t((N + 15) / 16) * 8));
+    // one record per 16 cells, ghosts included: the ghosts' blocks stay zero, as their states count
+    HIPCHK((hipError_t)trackAlloc(s, s->d_rmsBlocks, (C / 16 + 1) * 8));
     // the stage kernel's workgroup count: one (min dt, max |R|) pair each
     s->nPart = s->useTiles ? s->tiles.nBlocks : (s->useFaceTiles ? s->ftiles.nTiles : uint32_t((N + 255) / 256));
     s->pstride = 2 * uint32_t(std::max<size_t>({(N + 255) / 256, s->tiles.nBlocks, s->ftiles.nTiles})) + 2;
     HIPCHK((hipError_t)trackAlloc(s, s->d_partial, size_t(s->pstride) * 4));   // up to 4 stages per step
     HIPCHK((hipError_t)trackAlloc(s, s->d_hist, size_t(s->histCap) * HIST_FIELDS));
-    const uint64_t nb = uint64_t(C) / 16;
-    const uint64_t nchunks = (nb + RMS_CHUNK_BLOCKS - 1) / RMS_CHUNK_BLOCKS + 1;
-    HIPCHK((hipError_t)trackAlloc(s, s->d_chunkTrees, size_t(nchunks) * 128));
-    HIPCHK((hipError_t)trackAlloc(s, s->d_chunkMask, size_t(nchunks) * 8));
+    HIPCHK((hipError_t)trackAlloc(s, s->d_chunkTops, size_t(C / 16 / RMS_CHUNK_BLOCKS + 1) * 8));
+    {
+        bool tpin = false;
+        for (const BFace& bf : s->bfaces) tpin = tpin || bf.type == TempPresInflow;
+        s->rideEpilogue = s->rmsFused && !tpin;
+    }
+    if (s->rideEpilogue && !s->useGradTiles) HIPCHK((hipError_t)trackAlloc(s, s->d_ghostSave, s->G));
     HIPCHK(hipMalloc((void**)&s->d_sc, sizeof(DevScalars)));
     HIPCHK(hipHostMalloc((void**)&s->h_sc, sizeof(DevScalars), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void**)&s->h_hist, sizeof(double) * size_t(s->histCap) * HIST_FIELDS, hipHostMallocDefault));
@@ -1277,31 +1274,48 @@ int ebb_run(ebb_solver* s, int64_t max_steps, double* t, double* dt, int64_t* st
                 limit = (limit < 0) ? left : std::min(limit, left);
             }
             if (limit == 0) goto out;
-            s->h_sc->active = 1;
-            HIPCHK(hipMemcpyAsync(&s->d_sc->active, &s->h_sc->active, sizeof(int32_t), hipMemcpyHostToDevice, s->stream));
+            auto activate = [&]() -> int {
+                s->h_sc->active = s->h_sc->specActive = 1;   // adjacent
+                HIPCHK(hipMemcpyAsync(&s->d_sc->active, &s->h_sc->active, 2 * sizeof(int32_t), hipMemcpyHostToDevice,
+                                      s->stream));
+                return EBB_OK;
+            };
+            { int rc_ = activate(); if (rc_) return rc_; }
             while (limit < 0 || done < limit) {
                 const int64_t batch = limit < 0 ? s->histCap : std::min<int64_t>(s->histCap, limit - done);
                 const int64_t base = s->h_sc->steps;
                 beginErrorWindow(s);   // no error is pending: the previous batch would have stopped
                 const int64_t stopAt = base + batch;
                 int c0 = s->cur;
+                DiagArgs d{};
                 for (int64_t k = 0; k < batch; k++) {
                     const double4* qold = s->qcur();
-                    stepStages(s, 1, uint32_t(base + k));
-                    const double4* qnew = s->qnext();
-                    DiagArgs d = diagArgs(s, qnew, qold, base, stopAt);
-                    launchRmsChunks(d, s->stream);
-                    launchFinalize(d, s->stream);
+                    stepStages(s, 1, uint32_t(base + k), k && s->rideEpilogue ? &d : nullptr);
+                    d = diagArgs(s, s->qnext(), qold, base, stopAt);
+                    if (!s->rmsFused) launchRmsLeaves(d, s->d_rmsBlocks.p, s->stream);
+                    if (!s->rideEpilogue || k + 1 == batch) launchEpilogue(d, s->stream);
                     s->cur ^= 1;
                 }
-                // the batch's last step (or the one that ended the loop) still has its force pending
-                if (deferForce(s)) launchPendingForce(forceArgs(s), s->d_sc, s->stream);
                 HIPCHK(hipGetLastError());
                 HIPCHK(hipMemcpyAsync(s->h_hist, s->d_hist.p, sizeof(double) * size_t(batch) * HIST_FIELDS,
                                       hipMemcpyDeviceToHost, s->stream));
                 { int rc_ = readScalars(s); if (rc_) return rc_; }
                 const int64_t ran = s->h_sc->steps - base;
                 s->cur = (c0 ^ int(ran & 1));
+                if (ran < batch) {
+                    // the loop ended before the last launches queued: the last stage that ran read T,
+                    // or with one stage per step the buffer the ended loop's last step started from
+                    if (stagesPerStep(s->cfg) == 1) s->lastInput = s->qnext();
+                    if (s->rideEpilogue) {
+                        // the gradient kernel that carried the ending epilogue has replaced the ghost
+                        // rows of the final state and the gradients of the last stage
+                        s->gradStale = true;
+                        float4* q32 = shadowOf(s, s->qcur());
+                        if (s->d_ghostSave.p)
+                            launchRestoreGhosts(s->qcur() + s->N, q32 ? q32 + s->N : nullptr, s->d_ghostSave.p, s->G,
+                                                s->stream);
+                    }
+                }
                 s->history.insert(s->history.end(), s->h_hist, s->h_hist + ran * HIST_FIELDS);
                 s->stepsTotal += ran;
                 done += ran;
@@ -1309,8 +1323,7 @@ int ebb_run(ebb_solver* s, int64_t max_steps, double* t, double* dt, int64_t* st
                 if (rc != EBB_OK) break;
                 if (ran < batch) break;              // t >= tEnd
                 if (!(s->h_sc->t < s->cfg.tEnd)) break;
-                s->h_sc->active = 1;
-                HIPCHK(hipMemcpyAsync(&s->d_sc->active, &s->h_sc->active, sizeof(int32_t), hipMemcpyHostToDevice, s->stream));
+                { int rc_ = activate(); if (rc_) return rc_; }
             }
         }
     out:
@@ -1420,9 +1433,9 @@ int ebb_cell_gradients(ebb_solver* s, double* grad, double* lim)
     return guarded([&]() -> int {
         if (!s) return EBB_ERR_ARG;
         HIPCHK(hipSetDevice(s->device));
-        // the fused and gradient-tile kernels keep gradients in LDS: recompute them for the last
-        // stage input
-        if (s->useTiles || s->useGradTiles) { int rc_ = refreshEdgeStates(s); if (rc_) return rc_; }
+        // the fused and gradient-tile kernels keep gradients in LDS, and a loop that ended early has
+        // overwritten them: recompute them for the last stage input
+        if (s->useTiles || s->useGradTiles || s->gradStale) { int rc_ = refreshEdgeStates(s); if (rc_) return rc_; }
         if (grad) {
             int rc_ = s->phys.mixed ? downloadCellsF(s, s->d_grad32.p, grad, 8) : downloadCells(s, s->d_grad.p, grad, 8);
             if (rc_) return rc_;
@@ -1678,7 +1691,7 @@ void ebb_solver_destroy(ebb_solver* s)
     s->d_nbr.release(); s->d_cface.release(); s->d_refId.release(); s->d_forceFaces.release();
     s->d_nia.release(); s->d_cd.release(); s->d_cper.release(); s->d_flen.release();
     s->d_grad.release(); s->d_lim.release(); s->d_lenF.release(); s->d_lenS.release(); s->d_celldt.release();
-    s->d_hist.release(); s->d_chunkTrees.release(); s->d_chunkMask.release(); s->d_partial.release();
+    s->d_hist.release(); s->d_chunkTops.release(); s->d_ghostSave.release(); s->d_partial.release();
     s->d_cen.release(); s->d_fn.release(); s->d_fmid.release(); s->d_fcell.release(); s->d_bface.release();
     s->d_src.release(); s->d_qA.release(); s->d_qB.release(); s->d_T.release(); s->d_T2.release();
     s->d_acc.release(); s->d_R.release(); s->d_estate.release();

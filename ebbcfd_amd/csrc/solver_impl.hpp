@@ -88,13 +88,12 @@ struct ebb_solver {
     DevMesh dm{};
     // device buffers
     DBuf<uint32_t> d_nbr, d_cface, d_refId, d_forceFaces;
-    DBuf<double> d_nia, d_cd, d_cper, d_flen, d_grad, d_lim, d_lenF, d_lenS, d_celldt, d_hist, d_chunkTrees;
+    DBuf<double> d_nia, d_cd, d_cper, d_flen, d_grad, d_lim, d_lenF, d_lenS, d_celldt, d_hist, d_chunkTops;
     DBuf<double> d_partial;
     DBuf<double2> d_cen, d_fn, d_fmid;
     DBuf<uint2> d_fcell;
     DBuf<BFace> d_bface;
     DBuf<double4> d_src, d_qA, d_qB, d_T, d_T2, d_acc, d_R, d_estate;
-    DBuf<uint32_t> d_chunkMask;
     // mixed precision: FP32 shadows of the state buffers (paired with qA, qB, T, T2) and FP32
     // gradient and limiter rows
     DBuf<float4> d_qA32, d_qB32, d_T32, d_T232;
@@ -124,6 +123,11 @@ struct ebb_solver {
     // face tiles cut along aligned 16-cell blocks)
     bool rmsFused = false;
     DBuf<double> d_rmsBlocks;
+    // the epilogue of a step rides in the next step's first gradient kernel, which then runs before
+    // the loop is known to go on: not with a total-conditions inflow, whose ghost update may fail
+    bool rideEpilogue = false;
+    DBuf<double4> d_ghostSave;   // the ghost rows that gradient kernel replaced
+    bool gradStale = false;      // the loop ended under such a kernel: d_grad is not the last stage's
     DevScalars* d_sc = nullptr;
     DevScalars* h_sc = nullptr;  // pinned
     double* h_hist = nullptr;    // pinned
@@ -170,8 +174,6 @@ struct StageDesc {
 };
 std::vector<StageDesc> stepSequence(ebb_solver* s);
 DiagArgs diagArgs(ebb_solver* s, const double4* qnew, const double4* qold, int64_t histBase, int64_t maxSteps);
-ForceArgs forceArgs(const ebb_solver* s);
-bool deferForce(const ebb_solver* s);
 int stagesPerStep(const Config& c);
 void refreshShadow(ebb_solver* s);
 // the mixed-precision pointers of a stage reading qin and writing qout (null on the FP64 path)
