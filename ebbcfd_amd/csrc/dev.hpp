@@ -318,6 +318,8 @@ void launchGatherScalars(const MemberArgs* mem, const uint32_t* members, uint32_
                          hipStream_t stream);
 // ghost rows q[0..n) back from `save`, and their FP32 shadow (null on the FP64 path)
 void launchRestoreGhosts(double4* q, float4* q32, const double4* save, uint32_t n, hipStream_t stream);
+// out[i] = in[src[i]] for n rows of 4 doubles (device and reference numbering)
+void launchPermuteRows(const double4* in, double4* out, const uint32_t* src, uint32_t n, hipStream_t stream);
 // FP32 shadow q32[0..n) of q[0..n) (mixed precision)
 void launchShadow(const double4* q, float4* q32, uint32_t n, hipStream_t stream);
 

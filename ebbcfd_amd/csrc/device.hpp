@@ -1024,7 +1024,7 @@ DEV void cellStage(const DevMesh& m, const PhysParams& p, const StageArgs& a, ui
         else ld4(a.qn, i, qn);
     }
     if (KIND == SK_RESIDUAL) {
-        st4(a.R, i, R);
+        st4(a.R, m.refId[i], R);   // R is the caller's: reference numbering
     } else if (KIND == SK_EULER) {
 #pragma unroll
         for (int k = 0; k < 4; k++) o[k] = qn[k] + h * R[k];

@@ -214,6 +214,22 @@ void launchShadow(const double4* q, float4* q32, uint32_t n, hipStream_t st)
     if (n) hipLaunchKernelGGL(k_shadow, dim3((n + BLK - 1) / BLK), dim3(BLK), 0, st, q, q32, n);
 }
 
+// Rows of 4 doubles into another numbering: out[i] = in[src[i]], a lane per half row
+__global__ __launch_bounds__(BLK) void k_permute_rows(const double2* __restrict__ in, double2* __restrict__ out,
+                                                      const uint32_t* __restrict__ src, uint32_t n)
+{
+    const uint64_t g = uint64_t(blockIdx.x) * BLK + threadIdx.x;
+    const uint32_t i = uint32_t(g >> 1), h = uint32_t(g & 1u);
+    if (i < n) out[g] = in[size_t(src[i]) * 2 + h];
+}
+
+void launchPermuteRows(const double4* in, double4* out, const uint32_t* src, uint32_t n, hipStream_t st)
+{
+    if (n)
+        hipLaunchKernelGGL(k_permute_rows, dim3((2 * uint64_t(n) + BLK - 1) / BLK), dim3(BLK), 0, st,
+                           reinterpret_cast<const double2*>(in), reinterpret_cast<double2*>(out), src, n);
+}
+
 __global__ void k_init_scalars(DevScalars* sc, double dt, double t, double CFL)
 {
     sc->newDtBits = 0x7FF0000000000000ull;
