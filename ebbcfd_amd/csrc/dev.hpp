@@ -50,6 +50,7 @@ struct DevScalars {
     unsigned long long errBC;       // (stage << 32) | boundary face whose total-conditions inflow has no
                                     // non-negative Mach root (solve.d:648-671), min wins; ~0 = none
     double rms0;                    // rho RMS residual of the first step (convergence stop)
+    double loopDt;                  // the run loop's dt while a bare integrator step runs with the caller's
 };
 
 struct DevMesh {
@@ -297,6 +298,11 @@ void launchRmsLeaves(const DiagArgs& d, double* blockSums, hipStream_t stream);
 // the epilogue of a step as a launch of its own
 void launchEpilogue(const DiagArgs& d, hipStream_t stream);
 void launchInitScalars(DevScalars* sc, double dt, double t, double CFL, hipStream_t stream);
+
+// before a residual or step outside the run loop: Rmax starts from rmaxBits, the error words are
+// cleared, and the step's dt is *dt where given; launchEndCall puts the run loop's dt back
+void launchBeginCall(DevScalars* sc, unsigned long long rmaxBits, const double* dt, hipStream_t stream);
+void launchEndCall(DevScalars* sc, hipStream_t stream);
 
 // Batched launches over many meshes (one launch per kernel for all of them).  The kernel
 // shape (S, flux, viscous, order, limiter mode, precision) is the group's; items are

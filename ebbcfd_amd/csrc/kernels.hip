@@ -248,11 +248,26 @@ __global__ void k_init_scalars(DevScalars* sc, double dt, double t, double CFL)
     sc->ticket = 0;
     sc->converged = 0;
     sc->rms0 = 0;
+    sc->loopDt = 0;
     for (int v = 0; v < 4; v++) sc->rms[v] = 0;
     sc->force[0] = sc->force[1] = 0;
     sc->fsum[0] = sc->fsum[1] = 0;
     sc->stageSum[0] = sc->stageSum[1] = 0;
 }
+
+__global__ void k_begin_call(DevScalars* sc, unsigned long long rmaxBits, double dt, int setDt)
+{
+    sc->rmaxBits = rmaxBits;
+    sc->errEdge = ~0ull;
+    sc->errCell = ~0ull;
+    sc->errBC = ~0ull;
+    if (setDt) {
+        sc->loopDt = sc->dt;
+        sc->dt = dt;
+    }
+}
+
+__global__ void k_end_call(DevScalars* sc) { sc->dt = sc->loopDt; }
 
 // ---------------------------------------------------------------- launchers
 static uint32_t nblk(uint64_t n) { return uint32_t((n + BLK - 1) / BLK); }
@@ -332,6 +347,13 @@ void launchEpilogue(const DiagArgs& d, hipStream_t st)
 {
     hipLaunchKernelGGL(k_epilogue, dim3(d.nEpi), dim3(EPT), 0, st, d);
 }
+
+void launchBeginCall(DevScalars* sc, unsigned long long rmaxBits, const double* dt, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_begin_call, dim3(1), dim3(1), 0, st, sc, rmaxBits, dt ? *dt : 0.0, dt ? 1 : 0);
+}
+
+void launchEndCall(DevScalars* sc, hipStream_t st) { hipLaunchKernelGGL(k_end_call, dim3(1), dim3(1), 0, st, sc); }
 
 void launchInitScalars(DevScalars* sc, double dt, double t, double CFL, hipStream_t st)
 {

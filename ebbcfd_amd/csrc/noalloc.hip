@@ -43,17 +43,6 @@ int scratchFor(int device, double** out)
     return EBB_OK;
 }
 
-// Rmax starts from the caller's value (the reference max-accumulates it, solve.d:1117);
-// the error words are cleared for this evaluation.  A kernel, not a host copy, so the call
-// needs no synchronisation before its launches.
-__global__ void k_prep_residual(DevScalars* sc, unsigned long long rmaxBits)
-{
-    sc->rmaxBits = rmaxBits;
-    sc->errEdge = ~0ull;
-    sc->errCell = ~0ull;
-    sc->errBC = ~0ull;
-}
-
 }  // namespace
 
 extern "C" int ebb_residual_noalloc(ebb_solver* s, int limit, int dt_update, double* R_dev, double* new_dt,
@@ -75,7 +64,8 @@ extern "C" int ebb_residual_noalloc(ebb_solver* s, int limit, int dt_update, dou
         { int rc = scratchFor(s->device, &ptr); if (rc) return rc; }
         unsigned long long bits = 0;
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
-        hipLaunchKernelGGL(k_prep_residual, dim3(1), dim3(1), 0, s->stream, s->d_sc, bits);
+        // a kernel, not a host copy, so the call needs no synchronisation before its launches
+        launchBeginCall(s->d_sc, bits, nullptr, s->stream);
         // the split kernels of ebb_residual, with R to the caller's buffer and the partials in scratch
         StageArgs a{};
         a.qin = s->qcur(); a.qn = s->qcur(); a.qout = nullptr; a.acc = s->d_acc.p;

@@ -160,8 +160,7 @@ StageArgs loopStageArgs(ebb_solver* s, int kind, double4* qin, const double4* qn
 
 // one residual evaluation + stage update
 void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qout, int limit, int dtUpdate,
-           int first, int last, int checkActive, double4* R, double4* estate, uint32_t stepId,
-           const DiagArgs* epi = nullptr)
+           int first, int last, int checkActive, double4* R, uint32_t stepId, const DiagArgs* epi = nullptr)
 {
     const uint32_t stageId = s->stageCounter++;
     StageArgs a;
@@ -172,13 +171,14 @@ void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qo
         a = baseStageArgs(s, kind, qin, qn, qout, limit, dtUpdate, first, last, stageId, stepId);
     }
     a.R = R;
-    a.estate = estate;
     s->stageStep.push_back(stepId);
-    if (s->useTiles && !estate && kind != SK_RESIDUAL) {
+    // a bare residual (ebb_residual) leaves every cell's gradient row: the gradient kernel and the
+    // face tiles, or the split kernels where there are none
+    if (s->useTiles && kind != SK_RESIDUAL) {
         launchStageTiles(s->dm, s->phys, a, s->tiles, int(s->S), s->stream);
-    } else if (s->useGradTiles && !estate && kind != SK_RESIDUAL) {
+    } else if (s->useGradTiles && kind != SK_RESIDUAL) {
         launchGradTiles(s->dm, s->phys, a, s->ftiles, int(s->S), s->stream, 3, epi);
-    } else if (s->useFaceTiles && !estate && kind != SK_RESIDUAL) {
+    } else if (s->useFaceTiles) {
         launchGradient(s->dm, s->phys, a, int(s->S), s->stream, epi);
         launchFaceTiles(s->dm, s->phys, a, s->ftiles, int(s->S), s->stream);
     } else {
@@ -217,7 +217,7 @@ void stepStages(ebb_solver* s, int checkActive, uint32_t stepId, const DiagArgs*
     s->stageInStep = 0;
     const double4* q = s->qcur();
     for (const StageDesc& x : stepSequence(s)) {
-        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, nullptr, stepId, epi);
+        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, stepId, epi);
         epi = nullptr;
     }
 }
@@ -1218,23 +1218,16 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
     return guarded([&]() -> int {
         if (!s) return EBB_ERR_ARG;
         HIPCHK(hipSetDevice(s->device));
-        if (!s->d_R.p) HIPCHK((hipError_t)trackAlloc(s, s->d_R, s->N));
-        if (!s->d_estate.p) HIPCHK((hipError_t)trackAlloc(s, s->d_estate, size_t(s->Fi + s->Fb) * 2));
-        { int rc_ = readScalars(s); if (rc_) return rc_; }
-        s->h_sc->rmaxBits = 0;
-        if (rmax && *rmax > 0) std::memcpy(&s->h_sc->rmaxBits, rmax, 8);
+        { int rc_ = rowStaging(s); if (rc_) return rc_; }
+        unsigned long long bits = 0;
+        if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         beginErrorWindow(s);
-        s->h_sc->errEdge = ~0ull;
-        s->h_sc->errCell = ~0ull;
-        s->h_sc->errBC = ~0ull;
-        HIPCHK(hipMemcpyAsync(s->d_sc, s->h_sc, sizeof(DevScalars), hipMemcpyHostToDevice, s->stream));
-        stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, s->d_estate.p, 0);
+        launchBeginCall(s->d_sc, bits, nullptr, s->stream);
+        stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, 0);
         HIPCHK(hipGetLastError());
+        // the kernel leaves R in the reference numbering
+        if (R) HIPCHK(hipMemcpyAsync(R, s->d_R.p, size_t(s->N) * sizeof(double4), hipMemcpyDeviceToHost, s->stream));
         { int rc_ = readScalars(s); if (rc_) return rc_; }
-        if (R) {   // the kernel leaves R in the reference numbering
-            HIPCHK(hipMemcpyAsync(R, s->d_R.p, size_t(s->N) * sizeof(double4), hipMemcpyDeviceToHost, s->stream));
-            HIPCHK(hipStreamSynchronize(s->stream));
-        }
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);
         std::memcpy(&rm, &s->h_sc->rmaxBits, 8);
@@ -1249,15 +1242,11 @@ int ebb_step(ebb_solver* s, double* dt, double* rmax)
     return guarded([&]() -> int {
         if (!s || !dt) return EBB_ERR_ARG;
         HIPCHK(hipSetDevice(s->device));
-        { int rc_ = readScalars(s); if (rc_) return rc_; }
-        DevScalars saved = *s->h_sc;
-        s->h_sc->dt = *dt;
         beginErrorWindow(s);
-        s->h_sc->errEdge = ~0ull;
-        s->h_sc->errCell = ~0ull;
-        s->h_sc->errBC = ~0ull;
-        HIPCHK(hipMemcpyAsync(s->d_sc, s->h_sc, sizeof(DevScalars), hipMemcpyHostToDevice, s->stream));
+        // the step runs with the caller's dt; the run loop's own is put back behind it on the device
+        launchBeginCall(s->d_sc, 0, dt, s->stream);
         stepStages(s, 0, uint32_t(s->stepsTotal));
+        launchEndCall(s->d_sc, s->stream);
         HIPCHK(hipGetLastError());
         { int rc_ = readScalars(s); if (rc_) return rc_; }
         s->cur ^= 1;
@@ -1266,12 +1255,7 @@ int ebb_step(ebb_solver* s, double* dt, double* rmax)
         std::memcpy(&rm, &s->h_sc->rmaxBits, 8);
         *dt = nd;
         if (rmax) *rmax = rm;
-        int rc = checkErrors(s);
-        // the run loop's time/dt are not advanced by a bare integrator step
-        s->h_sc->dt = saved.dt;
-        HIPCHK(hipMemcpyAsync(s->d_sc, s->h_sc, sizeof(DevScalars), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-        return rc;
+        return checkErrors(s);
     });
 }
 
