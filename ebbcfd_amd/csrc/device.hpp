@@ -49,6 +49,76 @@ DEV R pressure(const R q[4])
 template <typename R>
 DEV R dmax(R a, R b) { return a < b ? b : a; }
 
+// Division by one denominator, several times.  FAST 0: IEEE division.  FAST 1: one refined
+// reciprocal per denominator and one Markstein correction per quotient (P. Markstein, IBM J. Res.
+// Dev. 34, 1990): the correctly rounded quotient, so the same bits, for normal denominators and
+// quotients that do not underflow.  A zero, subnormal or infinite denominator or an infinite
+// numerator gives NaN, which the flux carries to its caller (interiorFaceFast), who then takes
+// the IEEE form.  A quotient after the first costs 3 instructions instead of 11.
+template <int FAST, typename R>
+struct Div {
+    R b, r;
+    DEV Div() {}
+    DEV explicit Div(R d) : b(d), r(R(0))
+    {
+        if constexpr (FAST && sizeof(R) == 8) {
+            const R r0 = __builtin_amdgcn_rcp(b);
+            const R r1 = __builtin_fma(__builtin_fma(-b, r0, R(1)), r0, r0);
+            r = __builtin_fma(__builtin_fma(-b, r1, R(1)), r1, r1);
+        } else if constexpr (FAST) {
+            const R r0 = __builtin_amdgcn_rcpf(b);
+            r = __builtin_fmaf(__builtin_fmaf(-b, r0, R(1)), r0, r0);
+        }
+    }
+    DEV R operator()(R a) const
+    {
+        if constexpr (FAST && sizeof(R) == 8) {
+            const R q = a * r;
+            return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+        } else if constexpr (FAST) {
+            const R q = a * r;
+            const R q1 = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+            return __builtin_fmaf(__builtin_fmaf(-b, q1, a), r, q1);
+        } else {
+            return a / b;
+        }
+    }
+};
+
+// sqrt, with FAST 1 (FP64) by Goldschmidt's iteration from the hardware's reciprocal root without
+// the scaling that subnormal arguments need: the correctly rounded root, the same bits, for normal
+// arguments; NaN for zero and infinity, which takes the flux to its IEEE form like Div's.
+template <int FAST, typename R>
+DEV R root(R x)
+{
+    if constexpr (FAST && sizeof(R) == 8) {
+        const R y = __builtin_amdgcn_rsq(x);
+        R g = x * y, h = R(0.5) * y;
+        const R e = __builtin_fma(-h, g, R(0.5));
+        g = __builtin_fma(g, e, g);
+        h = __builtin_fma(h, e, h);
+        g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+        return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    } else {
+        return sqrt(x);
+    }
+}
+
+// A state's velocity and pressure, by the operations of pressure(), with the divider by its
+// density for the flux's further quotients.
+template <int FAST, typename R>
+struct Prim {
+    Div<FAST, R> rho;
+    R u, v, p;
+    DEV Prim() {}
+    DEV explicit Prim(const R q[4]) : rho(q[0])
+    {
+        u = rho(q[1]);
+        v = rho(q[2]);
+        p = R(G_ - 1) * (q[3] - R(0.5) * q[0] * (u * u + v * v));
+    }
+};
+
 template <typename R>
 DEV R harten(R lam, R eps)
 {
@@ -67,24 +137,23 @@ DEV void convective(R p, R u, R v, R rho, R e, R n0, R n1, R out[4])
 }
 
 // flux.d:224-303
-template <typename R>
-DEV void roeFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
+template <int FAST, typename R>
+DEV void roeFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1, R out[4],
+                 R& sMax)
 {
     const R gm1 = R(G_ - 1), half = R(0.5);
-    const R rhoL = qL[0], uL = qL[1] / rhoL, vL = qL[2] / rhoL;
+    const R rhoL = qL[0], uL = wL.u, vL = wL.v, pL = wL.p;
     const R rvL0 = rhoL * uL, rvL1 = rhoL * vL;
-    const R pL = (gm1 * (qL[3] - half * rhoL * (uL * uL + vL * vL)));
-    const R hL = (qL[3] + pL) / rhoL;
-    const R rhoR = qR[0], uR = qR[1] / rhoR, vR = qR[2] / rhoR;
+    const R hL = wL.rho(qL[3] + pL);
+    const R rhoR = qR[0], uR = wR.u, vR = wR.v, pR = wR.p;
     const R rvR0 = rhoR * uR, rvR1 = rhoR * vR;
-    const R pR = (gm1 * (qR[3] - half * rhoR * (uR * uR + vR * vR)));
-    const R hR = (qR[3] + pR) / rhoR;
-    const R di = sqrt(rhoR / rhoL);
-    const R d1 = R(1.0) / (R(1.0) + di);
+    const R hR = wR.rho(qR[3] + pR);
+    const R di = root<FAST, R>(wL.rho(rhoR));
+    const R d1 = Div<FAST, R>(R(1.0) + di)(R(1.0));
     const R vel0 = (di * uR + uL) * d1, vel1 = (di * vR + vL) * d1;
     const R u = vel0 * n0 + vel1 * n1;
     const R h = (di * hR + hL) * d1;
-    const R a = sqrt(R(G_ - 1.0) * (h - half * (vel0 * vel0 + vel1 * vel1)));
+    const R a = root<FAST, R>(R(G_ - 1.0) * (h - half * (vel0 * vel0 + vel1 * vel1)));
     const R dRhoV0 = rvR0 - rvL0, dRhoV1 = rvR1 - rvL1;
     const R dRho = rhoR - rhoL, dRhoE = qR[3] - qL[3];
     const R eps = R(0.01) * a;
@@ -97,8 +166,9 @@ DEV void roeFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
     const R qq = sqrt(vel0 * vel0 + vel1 * vel1);
     const R G1 = gm1 * (((qq * qq) / R(2.0)) * dRho - (vel0 * dRhoV0 + vel1 * dRhoV1) + dRhoE);
     const R G2 = -u * dRho + (dRhoV0 * n0 + dRhoV1 * n1);
-    const R C1 = (G1 / (a * a)) * (s1 - lam3) + G2 / a * s2;
-    const R C2 = (G1 / a) * s2 + (s1 - lam3) * G2;
+    const Div<FAST, R> byA(a), byA2(a * a);
+    const R C1 = byA2(G1) * (s1 - lam3) + byA(G2) * s2;
+    const R C2 = byA(G1) * s2 + (s1 - lam3) * G2;
     R fL[4], fR[4];
     convective<R>(pL, uL, vL, rhoL, qL[3], n0, n1, fL);
     convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
@@ -109,26 +179,26 @@ DEV void roeFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
 }
 
 // flux.d:66-141 (Roe-type averages, C1 = C2 = 0: central flux + sMax jump)
-template <typename R>
-DEV void rusanovFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
+// FAST 1 leaves out what the form with C1 = C2 = 0 multiplies by zero (s1 - sm and s2, with G1,
+// G2, h and the speed): the same bits as long as those factors are finite, that is unless the
+// sound speed vanishes; it then gives NaN as the full form does.
+template <int FAST, typename R>
+DEV void rusanovFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1,
+                     R out[4], R& sMax)
 {
-    const R gm1 = R(G_ - 1), half = R(0.5);
-    const R rhoL = qL[0], uL = qL[1] / rhoL, vL = qL[2] / rhoL;
+    const R half = R(0.5);
+    const R rhoL = qL[0], uL = wL.u, vL = wL.v, pL = wL.p;
     const R rvL0 = rhoL * uL, rvL1 = rhoL * vL;
-    const R pL = (gm1 * (qL[3] - half * rhoL * (uL * uL + vL * vL)));
-    const R hL = (qL[3] + pL) / rhoL;
-    const R rhoR = qR[0], uR = qR[1] / rhoR, vR = qR[2] / rhoR;
+    const R rhoR = qR[0], uR = wR.u, vR = wR.v, pR = wR.p;
     const R rvR0 = rhoR * uR, rvR1 = rhoR * vR;
-    const R pR = (gm1 * (qR[3] - half * rhoR * (uR * uR + vR * vR)));
-    const R hR = (qR[3] + pR) / rhoR;
-    const R rho = sqrt(rhoL * rhoR);
-    const R sL = sqrt(rhoL), sR = sqrt(rhoR);
-    const R vel0 = (sL * uL + sR * uR) / (sL + sR);
-    const R vel1 = (sL * vL + sR * vR) / (sL + sR);
+    const R rho = root<FAST, R>(rhoL * rhoR);
+    const R sL = root<FAST, R>(rhoL), sR = root<FAST, R>(rhoR);
+    const Div<FAST, R> mean(sL + sR);
+    const R vel0 = mean(sL * uL + sR * uR);
+    const R vel1 = mean(sL * vL + sR * vR);
     const R u = vel0 * n0 + vel1 * n1;
-    const R p = (sL * pL + sR * pR) / (sL + sR);
-    const R h = (sL * hL + sR * hR) / (sL + sR);
-    const R a = sqrt(R(G_) * (p / rho));
+    const R p = mean(sL * pL + sR * pR);
+    const R a = root<FAST, R>(R(G_) * Div<FAST, R>(rho)(p));
     const R dRhoV0 = rvR0 - rvL0, dRhoV1 = rvR1 - rvL1;
     const R dRho = rhoR - rhoL, dRhoE = qR[3] - qL[3];
     const R eps = R(0.01) * a;
@@ -138,37 +208,54 @@ DEV void rusanovFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax
     const R lam4 = harten<R>(fabs(u), eps);
     const R sm = dmax<R>(dmax<R>(dmax<R>(fabs(lam1), fabs(lam2)), fabs(lam3)), fabs(lam4));
     sMax = sm;
-    const R s1 = half * (sm + sm), s2 = half * (sm - sm);
-    const R qq = sqrt(vel0 * vel0 + vel1 * vel1);
-    const R G1 = gm1 * ((qq * qq / R(2)) * dRho - (vel0 * dRhoV0 + vel1 * dRhoV1) + dRhoE);
-    const R G2 = -u * dRho + (dRhoV0 * n0 + dRhoV1 * n1);
-    const R C1 = (G1 / (a * a)) * (s1 - sm) + G2 / a * s2;
-    const R C2 = (G1 / a) * s2 + (s1 - sm) * G2;
     R fL[4], fR[4];
     convective<R>(pL, uL, vL, rhoL, qL[3], n0, n1, fL);
     convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
-    const R d[4] = {sm * dRho + C1, sm * (dRhoV0) + C1 * vel0 + C2 * n0,
-                    sm * (dRhoV1) + C1 * vel1 + C2 * n1, sm * dRhoE + C1 * h + C2 * u};
+    R d[4];
+    if constexpr (FAST) {
+        const R z = a > R(sizeof(R) == 8 ? 1e-100 : 1e-12) ? sm : R(NAN);
+        d[0] = z * dRho; d[1] = z * dRhoV0; d[2] = z * dRhoV1; d[3] = z * dRhoE;
+    } else {
+        const R hL = wL.rho(qL[3] + pL), hR = wR.rho(qR[3] + pR);
+        const R h = (sL * hL + sR * hR) / (sL + sR);
+        const R s1 = half * (sm + sm), s2 = half * (sm - sm);
+        const R qq = sqrt(vel0 * vel0 + vel1 * vel1);
+        const R G1 = R(G_ - 1) * ((qq * qq / R(2)) * dRho - (vel0 * dRhoV0 + vel1 * dRhoV1) + dRhoE);
+        const R G2 = -u * dRho + (dRhoV0 * n0 + dRhoV1 * n1);
+        const R C1 = (G1 / (a * a)) * (s1 - sm) + G2 / a * s2;
+        const R C2 = (G1 / a) * s2 + (s1 - sm) * G2;
+        d[0] = sm * dRho + C1;
+        d[1] = sm * (dRhoV0) + C1 * vel0 + C2 * n0;
+        d[2] = sm * (dRhoV1) + C1 * vel1 + C2 * n1;
+        d[3] = sm * dRhoE + C1 * h + C2 * u;
+    }
 #pragma unroll
     for (int k = 0; k < 4; k++) out[k] = half * (fL[k] + fR[k]) - half * d[k];
 }
 
+template <int FLUX, int FAST, typename R>
+DEV void numFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1, R out[4],
+                 R& sMax)
+{
+    if (FLUX == 1) roeFlux<FAST, R>(qL, wL, qR, wR, n0, n1, out, sMax);
+    else rusanovFlux<FAST, R>(qL, wL, qR, wR, n0, n1, out, sMax);
+}
 template <int FLUX, typename R>
 DEV void numFlux(const R qL[4], const R qR[4], R n0, R n1, R out[4], R& sMax)
 {
-    if (FLUX == 1) roeFlux<R>(qL, qR, n0, n1, out, sMax);
-    else rusanovFlux<R>(qL, qR, n0, n1, out, sMax);
+    numFlux<FLUX, 0, R>(qL, Prim<0, R>(qL), qR, Prim<0, R>(qR), n0, n1, out, sMax);
 }
 
 // flux.d:28-64.  The four 4x4 matrices are applied entry by entry in column
 // order; their structural zeros only ever add a signed zero, so they are skipped.
 // Pr and mu are physical parameters (FP64), converted to R.
-template <typename R>
+template <typename R, int FAST = 0>
 DEV void viscousFlux(double Prd, double mud, const R q[4], const R dq[8], R n0, R n1, R out[4])
 {
-    const R rho = q[0], u = q[1] / q[0], v = q[2] / q[0], E = q[3] / q[0];
+    const Div<FAST, R> rho(q[0]);
+    const R u = rho(q[1]), v = rho(q[2]), E = rho(q[3]);
     const R gp = R(G_) / R(Prd);
-    const R s = R(mud) / rho;
+    const R s = rho(R(mud));
     const R one = R(1.0);
     const R c43 = R(4.0 / 3.0), c23 = R(2.0 / 3.0), cm43 = R(-4.0 / 3.0), cm23 = R(-2.0 / 3.0), c231 = R(2.0 / 3.0 - 1.0);
     const R t0 = (cm43 + gp) * (u * u) + (-one + gp) * (v * v) - gp * E;
@@ -466,8 +553,8 @@ DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t g
                 R s = R(1.0);
                 const R t = g[k][0] * dx + g[k][1] * dy;
                 const R qE = qi[k] + t;
-                if (qE < mn[k]) s = (mn[k] - qi[k]) / t;
-                else if (qE > mx[k]) s = (mx[k] - qi[k]) / t;
+                const bool under = qE < mn[k];
+                if (under || qE > mx[k]) s = ((under ? mn[k] : mx[k]) - qi[k]) / t;
                 lx[k] = fmin(lx[k], s);
                 ly[k] = lx[k];
             }
@@ -748,34 +835,41 @@ DEV void loadGrad(const float* grad, uint32_t c, float g[8])
     g[0] = a.x; g[1] = a.y; g[2] = a.z; g[3] = a.w; g[4] = b.x; g[5] = b.y; g[6] = b.z; g[7] = b.w;
 }
 
-// solve.d:980-1010 (interior) reconstruction with the p<0 fallback
-template <int LP, typename R>
-DEV void reconstruct(const R qm[4], const R g[8], const R lx[4], const R ly[4], R dx, R dy, R out[4])
+// solve.d:980-1010 (interior) reconstruction with the p<0 fallback; w: velocity and pressure of
+// the state that it arrives at
+template <int LP, int FAST, typename R>
+DEV void reconstruct(const R qm[4], const R g[8], const R lx[4], const R ly[4], R dx, R dy, R out[4],
+                     Prim<FAST, R>& w)
 {
 #pragma unroll
     for (int j = 0; j < 4; j++) out[j] = qm[j] + lx[j] * g[2 * j] * dx + ly[j] * g[2 * j + 1] * dy;
-    if (pressure<R>(out) < 0) {
+    w = Prim<FAST, R>(out);
+    if (w.p < 0) {
         R l0 = R(1.0), l1 = R(1.0);
 #pragma unroll
         for (int j = 0; j < 4; j++) { l0 = fmin(l0, lx[j]); l1 = fmin(l1, ly[j]); }
 #pragma unroll
         for (int j = 0; j < 4; j++) out[j] = qm[j] + l0 * g[2 * j] * dx + l1 * g[2 * j + 1] * dy;
+        w = Prim<FAST, R>(out);
     }
 }
 
 // solve.d:970-1033: one interior face from both cells' raw data.  Centroids, midpoint
 // and normal are FP64 geometry; the offsets and the normal enter the R arithmetic.
-template <int FLUX, int VISC, int ORDER, int LP, typename R>
+template <int FLUX, int VISC, int ORDER, int LP, typename R, int FAST = 0>
 DEV void interiorFace(const R qa[4], const R ga[8], const R lxa[4], const R lya[4], double2 ca,
                       const R qb[4], const R gb[8], const R lxb[4], const R lyb[4], double2 cb,
                       double2 n, double2 mid, const PhysParams& p, R qL[4], R qR[4], R F[4], R& sMax)
 {
+    Prim<FAST, R> wL, wR;
     if (ORDER > 1) {
-        reconstruct<LP, R>(qa, ga, lxa, lya, R(mid.x - ca.x), R(mid.y - ca.y), qL);
-        reconstruct<LP, R>(qb, gb, lxb, lyb, R(mid.x - cb.x), R(mid.y - cb.y), qR);
+        reconstruct<LP, FAST, R>(qa, ga, lxa, lya, R(mid.x - ca.x), R(mid.y - ca.y), qL, wL);
+        reconstruct<LP, FAST, R>(qb, gb, lxb, lyb, R(mid.x - cb.x), R(mid.y - cb.y), qR, wR);
     } else {
 #pragma unroll
         for (int k = 0; k < 4; k++) { qL[k] = qa[k]; qR[k] = qb[k]; }
+        wL = Prim<FAST, R>(qL);
+        wR = Prim<FAST, R>(qR);
     }
     // the face gradient is formed before the convective flux, so the two cell gradients
     // are not live across it
@@ -784,12 +878,12 @@ DEV void interiorFace(const R qa[4], const R ga[8], const R lxa[4], const R lya[
 #pragma unroll
         for (int k = 0; k < 8; k++) dq[k] = R(0.5) * (ga[k] + gb[k]);
     }
-    numFlux<FLUX, R>(qL, qR, R(n.x), R(n.y), F, sMax);
+    numFlux<FLUX, FAST, R>(qL, wL, qR, wR, R(n.x), R(n.y), F, sMax);
     if (VISC) {
         R qa2[4], Fv[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) qa2[k] = R(0.5) * (qL[k] + qR[k]);
-        viscousFlux<R>(p.Pr, p.mu, qa2, dq, R(n.x), R(n.y), Fv);
+        viscousFlux<R, FAST>(p.Pr, p.mu, qa2, dq, R(n.x), R(n.y), Fv);
 #pragma unroll
         for (int k = 0; k < 4; k++) F[k] = F[k] - Fv[k];
     }

@@ -13,13 +13,15 @@ namespace ebb {
 // of the mesh set-up (source/mesh.d; mesh.cpp), so they equal the stored ones bit
 // for bit.  Interior edges: normal = (y1-y0, x0-x1)/|.|, whose norm is the length
 // (the same squares summed in the other order); boundary edges: (1/len) * (...).
+template <int FAST = 0>
 DEV void edgeGeometry(bool interior, double2 p0, double2 p1, double2& n, double2& mid, double& len)
 {
     const double ddx = p0.x - p1.x, ddy = p0.y - p1.y;
-    len = sqrt(ddx * ddx + ddy * ddy);
+    len = root<FAST, double>(ddx * ddx + ddy * ddy);
     const double vx = p1.y - p0.y, vy = p0.x - p1.x;
     if (interior) {
-        n = make_double2(vx / len, vy / len);
+        const Div<FAST, double> byLen(len);
+        n = make_double2(byLen(vx), byLen(vy));
     } else {
         const double inv = 1.0 / len;
         n = make_double2(inv * vx, inv * vy);
@@ -161,6 +163,42 @@ DEV void tileCellPhase(const DevMesh& m, const PhysParams& p, const StageArgs& a
     blockPartial(dtCand, rCand, a.partial, pslot);
 }
 
+// Whether a face's flux by the FAST forms stands: every quotient outside their range (a zero,
+// subnormal or infinite denominator, a vanishing sound speed) has reached it as a NaN or as a
+// value beyond any flow's.  The forms with a guard on every quotient took longer than plain
+// divisions; this one test takes the 4.2M-cell viscous Rusanov launches from 295 to 265-278 us
+// (VALU issue was ~155 us of them) and a 299,266-cell Roe launch from 33.6 to 32.4 us.
+template <typename R>
+DEV bool fluxInRange(const R F[4])
+{
+    constexpr R big = sizeof(R) == 8 ? R(1e100) : R(1e30);
+    return fabs(F[0]) < big && fabs(F[1]) < big && fabs(F[2]) < big && fabs(F[3]) < big;
+}
+
+// An interior face by the IEEE forms, its rows loaded again: the fast path's registers do not
+// keep them for it (the opaque record stops the compiler from doing so).
+template <int FLUX, int VISC, int ORDER, int LP, int MIX>
+DEV void exactFace(const DevMesh& m, const PhysParams& p, const FaceSrc<MIX>& src, uint4 r,
+                   typename FaceSrc<MIX>::R F[4], typename FaceSrc<MIX>::R& sMax)
+{
+    using R = typename FaceSrc<MIX>::R;
+    asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z), "+v"(r.w));
+    double2 n, mid, ca = make_double2(0, 0), cb = make_double2(0, 0);
+    double len;
+    edgeGeometry(true, m.node[r.z], m.node[r.w], n, mid, len);
+    R qa[4], qb[4], ga[8], gb[8], lxa[4], lya[4], lxb[4], lyb[4], qL[4], qR[4];
+    src.q(r.x, qa);
+    src.q(r.y, qb);
+    if (ORDER > 1 || VISC) { src.grad(r.x, ga); src.grad(r.y, gb); }
+    if (ORDER > 1) {
+        src.template lim<LP>(r.x, lxa, lya);
+        src.template lim<LP>(r.y, lxb, lyb);
+        ca = m.cen[r.x];
+        cb = m.cen[r.y];
+    }
+    interiorFace<FLUX, VISC, ORDER, LP, R>(qa, ga, lxa, lya, ca, qb, gb, lxb, lyb, cb, n, mid, p, qL, qR, F, sMax);
+}
+
 // One workgroup of the face/update kernel on tile `tile` of its mesh, leaving its (min dt,
 // max |R|) pair in partial slot `pslot` (the solo and the batched kernels run this same code).
 template <int S, int FLUX, int VISC, int ORDER, int LP, int MIX>
@@ -205,13 +243,14 @@ DEV void faceTileBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
         }
         double2 n, mid;
         double len;
-        edgeGeometry(interior, p0, p1, n, mid, len);
+        edgeGeometry<1>(interior, p0, p1, n, mid, len);
         R qL[4], qR[4], Fr[4], sMr;
         bool isB = false;
         uint32_t b = 0;
         if (interior) {
-            interiorFace<FLUX, VISC, ORDER, LP, R>(qa, ga, lxa, lya, ca, qb, gb, lxb, lyb, cb, n, mid, p, qL, qR, Fr,
-                                                  sMr);
+            interiorFace<FLUX, VISC, ORDER, LP, R, 1>(qa, ga, lxa, lya, ca, qb, gb, lxb, lyb, cb, n, mid, p, qL, qR,
+                                                     Fr, sMr);
+            if (!fluxInRange(Fr)) exactFace<FLUX, VISC, ORDER, LP, MIX>(m, p, src, r, Fr, sMr);
         } else {
             isB = true;
             b = r.y - m.N;   // the ghost of boundary face b is cell N + b
