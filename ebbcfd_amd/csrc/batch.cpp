@@ -146,8 +146,9 @@ int followSpread(ebb_batch* b)
     for (auto& mb : b->members) {
         ebb_solver* s = mb.s;
         if (!mb.running || s->cfg.tileCells != -1 || !s->cfg.spreadTiles) continue;
-        const uint32_t was = spreadTileCells(uint64_t(s->N) + uint64_t(std::max<int64_t>(s->cfg.spreadOver, 0)), s->cus);
-        const uint32_t now = spreadTileCells(uint64_t(total), s->cus);
+        const uint32_t was = spreadTileCells(s->N, uint64_t(std::max<int64_t>(s->cfg.spreadOver, 0)), s->cus,
+                                             uint32_t(s->S), s->cfg);
+        const uint32_t now = spreadTileCells(s->N, uint64_t(total) - s->N, s->cus, uint32_t(s->S), s->cfg);
         if (now <= 2 * was && was <= 2 * now) continue;
         s->cfg.spreadOver = total - int64_t(s->N);
         int rc = retileFaceTiles(s, -1);

@@ -319,12 +319,32 @@ int clearErrors(ebb_solver* s)
     return EBB_OK;
 }
 
-// Down to 32 cells, in whole 16-cell blocks: a tile's workgroup takes about the same time
-// for any tile size up to one round of lanes, so smaller tiles only buy more workgroups.
-uint32_t spreadTileCells(uint64_t cells, int cus)
+// Automatic tile size of a launch over `cells` cells, in whole 16-cell blocks from 32 to 768: the
+// tiles fill a whole number of rounds over the CUs.  A tile whose faces fit one round of a
+// workgroup's lanes takes about the same time whatever its size, so one tile per CU, or two, are
+// best as long as they fit; larger tiles take as many per CU as stay resident (3, or 4 in mixed
+// precision; more tiles than that leave a tail).  Rounding the size up keeps the count from
+// spilling into one more round.  us per run, one / two / three / four tiles per CU: 30,976 viscous
+// triangles 1506 / 1558 / 1607 / 1895, 44,944: 1840 / 1701 / 1729 / 1948, 99,856: 2504 / 2289 /
+// 2236 / 2393, 299,266 inviscid triangles - / 4214 / 4164 / 4563, 59,784 quadrilaterals 2965 / 2937
+// / 2811 / 2987; mixed precision, 349,184 quadrilaterals - / 4542 / 4380 / 4259.  The rule before
+// (two per CU, rounded down) took 4608 us on the 299,266 triangles.  Gradient tiles and batched
+// members beside others keep that rule: a group's launches hold tiles of many meshes, whose short
+// ones spoil whole rounds, and the smaller sizes had more members cut again as a batch fills (the
+// first pass of 24 members 29 instead of 22 ms, for the same steps).
+uint32_t spreadTileCells(uint64_t own, uint64_t others, int cus, uint32_t S, const Config& c)
 {
-    const uint64_t share = cells / (2 * uint64_t(std::max(cus, 1))) / 16 * 16;
-    return uint32_t(std::max<uint64_t>(32, std::min<uint64_t>(768, share)));
+    const uint64_t cu = uint64_t(std::max(cus, 1)), cells = own + others;
+    if (c.stagePath == 3 || others)
+        return uint32_t(std::max<uint64_t>(32, std::min<uint64_t>(768, cells / (2 * cu) / 16 * 16)));
+    auto share = [&](uint64_t perCu) { return std::max<uint64_t>(32, (cells + perCu * cu * 16 - 1) / (perCu * cu * 16) * 16); };
+    // faces of a tile of T cells: half its cells' edges and those along its outline
+    auto oneRound = [&](uint64_t T) {
+        return 0.5 * double(S * T) + 2.6 * double(S - 2) * std::sqrt(double(T)) <= double(FACE_TILE_LANES);
+    };
+    for (uint64_t perCu = 1; perCu <= 2; perCu++)
+        if (oneRound(share(perCu))) return uint32_t(share(perCu));
+    return uint32_t(std::min<uint64_t>(768, share(c.precision ? 4 : 3)));
 }
 
 // Tiled paths: choose the tile size (tileCells, or automatically: 768 cells per
@@ -346,10 +366,10 @@ int planTiles(ebb_solver* s, Layout& ref, Layout& lay, std::vector<uint32_t>& st
     std::vector<uint32_t> order;
     uint32_t T = want > 0 ? uint32_t(want) : (c.stagePath == 1 || c.stagePath == 3 ? 768 : 128);
     if (want <= 0 && c.spreadTiles && (c.stagePath == 1 || c.stagePath == 3)) {
-        // a mesh too small to give every CU two tiles of 768 cells gets smaller tiles, so it
+        // a mesh too small for a full residency of 768-cell tiles gets smaller ones, so it
         // still spreads over the GPU.  A batched member counts the cells running beside it:
         // the launches are shared
-        T = std::min(T, spreadTileCells(uint64_t(ref.N) + uint64_t(std::max<int64_t>(c.spreadOver, 0)), s->cus));
+        T = std::min(T, spreadTileCells(ref.N, uint64_t(std::max<int64_t>(c.spreadOver, 0)), s->cus, ref.S, c));
     }
     if (c.stagePath == 3 && want <= 0) {
         // automatic gradient tiles: the largest multiple of 16 up to 768 cells whose busiest
@@ -546,9 +566,9 @@ int64_t estimateDeviceBytes(const BuiltMesh& b, const Config& c)
     // gradient tiles: an LDS-row pair per face record, each tile's ring and the border (~0.3 N each)
     if (c.stagePath == 3) bytes += int64_t(1.7 * double(N)) * 4 + int64_t(0.6 * double(N)) * 4 + int64_t(1.1 * double(N)) * 4 * S + 4096;
     bytes += (C / 16 + 1) * 64;                            // RMS leaf sums
-    // tiles: ~700 cells each, or at least two per CU on small meshes (down to 32 cells)
+    // tiles: ~700 cells each, or up to four per CU on small meshes (down to 32 cells)
     const int64_t tiles = std::max<int64_t>(N / (c.stagePath == 3 ? 250 : 700) + 1,
-                                            c.spreadTiles ? std::min<int64_t>(N / 32 + 1, 512) : 0);
+                                            c.spreadTiles ? std::min<int64_t>(N / 32 + 1, 1024) : 0);
     bytes += (2 * std::max<int64_t>((N + 255) / 256, tiles) + 2) * 4 * 8;   // stage partials
     bytes += 256 * HIST_FIELDS * 8;
     bytes += (C / 16 / RMS_CHUNK_BLOCKS + 1) * 64 + G * 32;   // chunk tops; ghost rows kept for a loop that ends

@@ -184,8 +184,9 @@ int checkErrors(ebb_solver* s);
 int64_t estimateDeviceBytes(const BuiltMesh& b, const Config& c);
 // face tiles cut again with tileCells per tile (batched runs' tuning)
 int retileFaceTiles(ebb_solver* s, long long tileCells);
-// automatic face-tile size that spreads `cells` over two tiles per CU (16-cell blocks, 32-768)
-uint32_t spreadTileCells(uint64_t cells, int cus);
+// automatic tile size that spreads a mesh's cells, with those of the `others` that share its
+// launches, over whole rounds of the CUs (16-cell blocks, 32-768)
+uint32_t spreadTileCells(uint64_t own, uint64_t others, int cus, uint32_t S, const Config& c);
 int fail(ebb_solver* s, int code, const std::string& msg);
 // creates a solver (ufvmSetup + upload) as ebb_solver_create does, with config overrides applied
 int createSolver(const ebb_mesh* m, const Config& c, int device, ebb_solver** out);
