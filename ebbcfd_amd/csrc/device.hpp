@@ -1075,26 +1075,36 @@ DEV void storeOut(const StageArgs& a, uint32_t i, const double o[4])
     if (a.qout32) a.qout32[i] = make_float4(float(o[0]), float(o[1]), float(o[2]), float(o[3]));
 }
 
+// Whether a stage's CFL time step is used: the last stage's is the step's (every stage overwrites
+// it in the reference), a residual call returns its own, and local time steps keep theirs.
+DEV bool stageWantsDt(const PhysParams& p, const StageArgs& a)
+{
+    return a.last || a.kind == SK_RESIDUAL || (p.localTimestep && a.dtUpdate);
+}
+
+// wantDt 0: sAve and the first two entries of met are not there
 template <int KIND>
 DEV void cellStage(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t i, const double r[4],
                    double sAve, const double* qinI, const double* met, double& dtCand, double& rCand,
                    double* qNew = nullptr, double* qOld = nullptr, const double* qnI = nullptr,
-                   const double* accI = nullptr)
+                   const double* accI = nullptr, bool wantDt = true)
 {
     auto loadAcc = [&](double v[4]) {
         if (accI) { v[0] = accI[0]; v[1] = accI[1]; v[2] = accI[2]; v[3] = accI[3]; }
         else ld4(a.acc, i, v);
     };
-    const double cper = met ? met[0] : m.cper[i], cd = met ? met[1] : m.cd[i], nia = met ? met[2] : m.nia[i];
-    sAve /= cper;
-    const double CFL = a.sc->CFL;
-    const double dtc = (CFL * cd) / sAve;
-    if (!isnan(dtc)) dtCand = fmin(dtCand, dtc);
+    const double nia = met ? met[2] : m.nia[i];
+    double dtc = 0.0;
+    if (wantDt) {
+        const double cper = met ? met[0] : m.cper[i], cd = met ? met[1] : m.cd[i];
+        sAve /= cper;
+        dtc = (a.sc->CFL * cd) / sAve;
+        if (!isnan(dtc)) dtCand = fmin(dtCand, dtc);
+    }
     double hc = 0.0;
     if (p.localTimestep) {
         if (a.dtUpdate) {
-            hc = CFL * cd / sAve;
-            if (isnan(hc)) hc = 0;
+            hc = isnan(dtc) ? 0.0 : dtc;
             a.celldt[i] = hc;
         } else {
             hc = a.celldt[i];
