@@ -1119,7 +1119,7 @@ static int uploadStates(ebb_solver* s, const double* host, double4* dev)
         { int rc_ = rowStaging(s); if (rc_) return rc_; }
         dst = s->d_R.p;
     }
-    HIPCHK(hipMemcpyAsync(dst, host, size_t(s->N) * sizeof(double4), hipMemcpyHostToDevice, s->stream));
+    HIPCHK(copyRows(s, const_cast<double*>(host), dst, size_t(s->N) * sizeof(double4), false));
     if (dst != dev) launchPermuteRows(dst, dev, s->d_refId.p, s->N, s->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1136,7 +1136,7 @@ static int downloadStates(ebb_solver* s, const double4* dev, double* host)
         HIPCHK(hipGetLastError());
         src = s->d_R.p;
     }
-    HIPCHK(hipMemcpyAsync(host, src, size_t(s->N) * sizeof(double4), hipMemcpyDeviceToHost, s->stream));
+    HIPCHK(copyRows(s, host, const_cast<double4*>(src), size_t(s->N) * sizeof(double4), true));
     HIPCHK(hipStreamSynchronize(s->stream));
     return EBB_OK;
 }
@@ -1246,7 +1246,7 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
         stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, 0);
         HIPCHK(hipGetLastError());
         // the kernel leaves R in the reference numbering
-        if (R) HIPCHK(hipMemcpyAsync(R, s->d_R.p, size_t(s->N) * sizeof(double4), hipMemcpyDeviceToHost, s->stream));
+        if (R) HIPCHK(copyRows(s, R, s->d_R.p, size_t(s->N) * sizeof(double4), true));
         { int rc_ = readScalars(s); if (rc_) return rc_; }
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);

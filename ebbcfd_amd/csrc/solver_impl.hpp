@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <exception>
 #include <new>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -73,6 +74,8 @@ struct DBuf {
 
 }  // namespace ebb
 
+namespace ebb { struct StagePool; }
+
 struct ebb_solver {
     // host copies
     RawMesh raw;
@@ -80,6 +83,7 @@ struct ebb_solver {
     Config cfg;
     int device = 0;
     hipStream_t stream = nullptr;
+    std::shared_ptr<ebb::StagePool> stagePool;   // page-locked slots of copyRows, from the first one that needs them
     uint32_t N = 0, G = 0, Fi = 0, Fb = 0, S = 3;
     std::vector<uint32_t> faceOfEdge;   // reference edge -> device face
     std::vector<uint32_t> edgeOfFace;   // device face -> reference edge
@@ -187,6 +191,9 @@ int retileFaceTiles(ebb_solver* s, long long tileCells);
 // automatic tile size that spreads a mesh's cells, with those of the `others` that share its
 // launches, over whole rounds of the CUs (16-cell blocks, 32-768)
 uint32_t spreadTileCells(uint64_t own, uint64_t others, int cus, uint32_t S, const Config& c);
+// `bytes` between device rows and the caller's memory on the solver's stream; from page-locked memory and
+// for small copies only enqueued, else done on return (an upload's slots included)
+hipError_t copyRows(ebb_solver* s, void* host, void* dev, size_t bytes, bool toHost);
 int fail(ebb_solver* s, int code, const std::string& msg);
 // creates a solver (ufvmSetup + upload) as ebb_solver_create does, with config overrides applied
 int createSolver(const ebb_mesh* m, const Config& c, int device, ebb_solver** out);

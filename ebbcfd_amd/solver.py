@@ -166,7 +166,7 @@ class Solver:
     # state
     @property
     def q(self):
-        out = np.zeros((self.n_interior, 4))
+        out = np.empty((self.n_interior, 4))
         _check(lib().ebb_state_download(self.h, _p(out)), "state download", self.h)
         return out
 
@@ -176,7 +176,7 @@ class Solver:
         _check(lib().ebb_state_upload(self.h, _p(v)), "state upload", self.h)
 
     def q_all(self):
-        out = np.zeros((self.n_cells, 4))
+        out = np.empty((self.n_cells, 4))
         _check(lib().ebb_state_download_all(self.h, _p(out)), "state download", self.h)
         return out
 
@@ -184,7 +184,7 @@ class Solver:
     def ufvm_solver(self, limit=True, dt_update=True, rmax=0.0, out=None):
         """One residual evaluation; returns (R, newDt, Rmax).  `out`: an n_interior x 4
         float64 array to receive R (e.g. a pinned_array), else a new one."""
-        R = np.zeros((self.n_interior, 4)) if out is None else out
+        R = np.empty((self.n_interior, 4)) if out is None else out
         if R.shape != (self.n_interior, 4) or R.dtype != np.float64 or not R.flags.c_contiguous:
             raise ValueError("out must be a C-contiguous float64 array of shape (%d, 4)" % self.n_interior)
         nd, rm = C.c_double(0), C.c_double(rmax)
@@ -339,7 +339,7 @@ class Batch:
         return dict(zip(BATCH_STATUS, out.tolist()))
 
     def q(self, sid):
-        out = np.zeros((self.meshes[sid].n_interior, 4))
+        out = np.empty((self.meshes[sid].n_interior, 4))
         _check(lib().ebb_batch_state_download(self.h, int(sid), _p(out)), "batch state")
         return out
 
