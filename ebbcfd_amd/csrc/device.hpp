@@ -479,10 +479,11 @@ DEV void lsqWeights(double2 ci, const double2 cn[S], double w[2][S])
 // the unlimited increment t = grad . (x_j - x_i) and the bound difference d = max - q_i (t > 0)
 // or min - q_i (t < 0), phi_j = [(d^2 + eps2) t + 2 t^2 d] / (t [d^2 + 2 t^2 + d t + eps2]),
 // phi = min(1, min_j phi_j); eps2 = (K d_cell)^3 (FP64, passed in).
-template <int S, int MODE, typename R>
-DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t gstride, double2 ci,
-                   const double2 cn[S], const bool real[S], int limit, double lpThresh, R g[4][2], R lx[4],
-                   R ly[4], double eps2d = 0.0)
+// V: the variables of this lane (all four, or one of them: each is independent of the others).
+template <int S, int MODE, typename R, int V = 4>
+DEV void gradLimit(const R qi[V], const R qn[S][V], const double* gm, uint32_t gstride, double2 ci,
+                   const double2 cn[S], const bool real[S], int limit, double lpThresh, R g[V][2], R lx[V],
+                   R ly[V], double eps2d = 0.0)
 {
     static_assert(MODE != 3 || sizeof(R) == 8, "the LP vector limiter runs in FP64 only");
     R w[2][S];
@@ -501,19 +502,19 @@ DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t g
 #pragma unroll
             for (int j = 0; j < S; j++) w[r][j] = R(wd[r][j]);
     }
-    R mn[4], mx[4], du[4][S];
+    R mn[V], mx[V], du[V][S];
 #pragma unroll
-    for (int k = 0; k < 4; k++) { mn[k] = qi[k]; mx[k] = qi[k]; }
+    for (int k = 0; k < V; k++) { mn[k] = qi[k]; mx[k] = qi[k]; }
 #pragma unroll
     for (int j = 0; j < S; j++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < V; k++) {
             mn[k] = fmin(mn[k], qn[j][k]);
             mx[k] = fmax(mx[k], qn[j][k]);
             du[k][j] = qn[j][k] - qi[k];
         }
 #pragma unroll
-    for (int k = 0; k < 4; k++)
+    for (int k = 0; k < V; k++)
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             R s = R(0.0);
@@ -522,14 +523,14 @@ DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t g
             g[k][r] = s;
         }
 #pragma unroll
-    for (int k = 0; k < 4; k++) { lx[k] = R(1.0); ly[k] = R(1.0); }
+    for (int k = 0; k < V; k++) { lx[k] = R(1.0); ly[k] = R(1.0); }
     if (MODE == 4 && limit) {
         const R eps2 = R(eps2d), two = R(2.0);
 #pragma unroll
         for (int j = 0; j < S; j++) {
             const R dx = R(cn[j].x - ci.x), dy = R(cn[j].y - ci.y);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
+            for (int k = 0; k < V; k++) {
                 const R t = g[k][0] * dx + g[k][1] * dy;
                 R s = R(1.0);
                 if (t != R(0.0)) {
@@ -549,7 +550,7 @@ DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t g
             const R dx = R(cn[j].x - ci.x), dy = R(cn[j].y - ci.y);
             dxs[j] = dx; dys[j] = dy;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
+            for (int k = 0; k < V; k++) {
                 R s = R(1.0);
                 const R t = g[k][0] * dx + g[k][1] * dy;
                 const R qE = qi[k] + t;
@@ -566,23 +567,27 @@ DEV void gradLimit(const R qi[4], const R qn[S][4], const double* gm, uint32_t g
                 for (int j = 0; j < S; j++) nn += real[j] ? 1 : 0;
                 // one copy of the simplex's code for the four variables, whose values are
                 // selected instead of indexed (an indexed array would live in scratch)
-                auto sel = [](int k, double v0, double v1, double v2, double v3) {
-                    return k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : v3;
+                auto sel = [](int k, const double v[V]) {
+                    if constexpr (V == 4) return k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+                    else return v[0];
                 };
+                double g0s[V], g1s[V];
+#pragma unroll
+                for (int k = 0; k < V; k++) { g0s[k] = g[k][0]; g1s[k] = g[k][1]; }
 #pragma unroll 1
-                for (int k = 0; k < 4; k++) {
-                    if (!(sel(k, lx[0], lx[1], lx[2], lx[3]) < lpThresh && (nn == 3 || nn == 4))) continue;
-                    const double g0 = sel(k, g[0][0], g[1][0], g[2][0], g[3][0]);
-                    const double g1 = sel(k, g[0][1], g[1][1], g[2][1], g[3][1]);
-                    const double q = sel(k, qi[0], qi[1], qi[2], qi[3]);
+                for (int k = 0; k < V; k++) {
+                    if (!(sel(k, lx) < lpThresh && (nn == 3 || nn == 4))) continue;
+                    const double g0 = sel(k, g0s);
+                    const double g1 = sel(k, g1s);
+                    const double q = sel(k, qi);
                     double ex[S], ey[S];
 #pragma unroll
                     for (int j = 0; j < S; j++) { ex[j] = dxs[j] * g0; ey[j] = dys[j] * g1; }
                     double x = 0.0, y = 0.0;
-                    lpSolve<S>(ex, ey, real, sel(k, mn[0], mn[1], mn[2], mn[3]) - q, q - sel(k, mx[0], mx[1], mx[2], mx[3]),
+                    lpSolve<S>(ex, ey, real, sel(k, mn) - q, q - sel(k, mx),
                                -fabs(g0), -fabs(g1), x, y);
 #pragma unroll
-                    for (int c = 0; c < 4; c++) {
+                    for (int c = 0; c < V; c++) {
                         lx[c] = c == k ? x : lx[c];
                         ly[c] = c == k ? y : ly[c];
                     }
@@ -611,7 +616,7 @@ DEV bool ghostFromOwner(const BFace& bf, const double qo[4], const double4* qbuf
 // LDS of one gradient workgroup: staging of the gradient rows and of the limiter rows
 template <int MODE>
 struct GradLds {
-    static constexpr int LWS = MODE == 3 ? 8 : ((MODE == 2 || MODE == 4) ? 4 : 0);
+    static constexpr int LWS = (MODE == 2 || MODE == 4) ? 4 : 0;
     double sg[BLK][9];
     double sl[BLK][LWS + 1];
 };
@@ -702,7 +707,7 @@ DEV bool fluxRuns(const StageArgs& a, bool first)
 }
 
 // One workgroup of the gradient kernel on cell block `bid` of its mesh (the solo and the
-// batched kernels run this same code).
+// batched kernels run this same code).  Not MODE 3: the LP limiter runs in gradientQuadBody.
 template <int S, int MODE, int MIX>
 DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid, GradLds<MODE>& L)
 {
@@ -770,10 +775,7 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
         if (have) {
 #pragma unroll
             for (int c = 0; c < 4; c++) { sg[tid][2 * c] = g[c][0]; sg[tid][2 * c + 1] = g[c][1]; }
-            if (MODE == 3) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) { sl[tid][2 * c] = lx[c]; sl[tid][2 * c + 1] = ly[c]; }
-            } else if (MODE == 2 || MODE == 4) {
+            if (MODE == 2 || MODE == 4) {
 #pragma unroll
                 for (int c = 0; c < 4; c++) sl[tid][c] = lx[c];
             }
@@ -789,6 +791,71 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     }
     // MODE 1 (unlimited stage): every limiter is 1; the face kernels take LP = 2 and read none
 }
+
+// One workgroup of the gradient kernel with four lanes per cell, one per variable, on block `bid` of
+// BLK / 4 cells: the variables' gradients, bounds and limiters do not depend on each other (a boundary
+// cell's lanes each form the whole ghost state), and a cell's row of four is still one access.  Four
+// times the workgroups with a shorter chain each, for meshes that leave the chip idle.
+template <int S, int MODE, int MIX>
+DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid)
+{
+    using R = RealOf<MIX>;
+    if (!stageRuns(a)) return;
+    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;   // Rmax is per step
+    const uint32_t i = bid * (BLK / 4) + threadIdx.x / 4, v = threadIdx.x & 3u;
+    if (i >= m.N) return;
+    const R* rows;
+    if constexpr (MIX == 1) rows = reinterpret_cast<const R*>(a.qin32);
+    else rows = reinterpret_cast<const R*>(a.qin);
+    uint32_t nb[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) nb[j] = m.nbr[size_t(i) * S + j];
+    R qi[1] = {rows[size_t(i) * 4 + v]}, qn[S][1];
+    double2 cn[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) { qn[j][0] = rows[size_t(nb[j]) * 4 + v]; cn[j] = m.cen[nb[j]]; }
+    const double2 ci = m.cen[i];
+#pragma unroll
+    for (int j = 0; j < S; j++)
+        if (nb[j] >= m.N) {   // as in cellGradient; the first lane stores
+            const uint32_t b = nb[j] - m.N;
+            const BFace& bf = m.bface[b];
+            R qo[4], qg[4], was[4], old[4] = {0, 0, 0, 0};
+            ldStage<MIX>(a, i, qo);
+            ldStage<MIX>(a, nb[j], was);
+            if (bf.type == BT_TPIN) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) old[k] = was[k];
+            }
+            const bool ok = ghostState<R>(bf, qo, qg, old);
+            if (v == 0) {
+                if (a.ghostSave) a.ghostSave[b] = make_double4(was[0], was[1], was[2], was[3]);
+                if (!ok && a.recordErrors) atomicMin(&a.sc->errBC, (uint64_t(a.stageId) << 32) | b);
+                stGhostRow<MIX>(a, nb[j], qg);
+            }
+            qn[j][0] = v == 0 ? qg[0] : v == 1 ? qg[1] : v == 2 ? qg[2] : qg[3];
+        }
+    bool real[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) real[j] = nb[j] != i;
+    double eps2 = 0.0;
+    if constexpr (MODE == 4) {
+        const double kd = p.venkatK * m.cd[i];
+        eps2 = kd * kd * kd;
+    }
+    R g[1][2], lx[1], ly[1];
+    gradLimit<S, MODE, R, 1>(qi, qn, nullptr, 0, ci, cn, real, a.limit, p.lpThresh, g, lx, ly, eps2);
+    const size_t o = size_t(i) * 4 + v;
+    if constexpr (MIX == 1) {
+        reinterpret_cast<float2*>(a.grad32)[o] = make_float2(g[0][0], g[0][1]);
+        if (MODE == 2 || MODE == 4) a.lim32[o] = lx[0];
+    } else {
+        reinterpret_cast<double2*>(a.grad)[o] = make_double2(g[0][0], g[0][1]);
+        if (MODE == 3) reinterpret_cast<double2*>(a.lim)[o] = make_double2(lx[0], ly[0]);
+        else if (MODE == 2 || MODE == 4) a.lim[o] = lx[0];
+    }
+}
+
 // ---------------------------------------------------------------- faces
 // LP 0: scalar limiter (4 per cell); 1: LP vector limiter (x,y pairs); 2: an
 // unlimited stage, every limiter 1 (1*g is exactly g, so the products round as with

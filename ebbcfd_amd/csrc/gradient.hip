@@ -32,6 +32,18 @@ __global__ __launch_bounds__(BLK) void k_gradient(DevMesh m, PhysParams p, Stage
 }
 
 template <int S, int MODE, int MIX>
+__global__ __launch_bounds__(BLK) void k_gradient_quad(DevMesh m, PhysParams p, StageArgs a, DiagArgs d, uint32_t epiPad)
+{
+    __shared__ GradShared<0> L;   // the epilogue's
+    if (blockIdx.x < epiPad) {
+        if (blockIdx.x < d.nEpi) epilogueBody(d, blockIdx.x, L.x.e, L.x.staging);
+        return;
+    }
+    const uint32_t b = blockIdx.x - epiPad, nb = gridDim.x - epiPad;
+    gradientQuadBody<S, MODE, MIX>(m, p, a, (a.order & 2) ? xcdBlockBack(b, nb) : xcdBlock(b, nb));
+}
+
+template <int S, int MODE, int MIX>
 __global__ __launch_bounds__(BLK) void k_gradient_batch(const MemberArgs* __restrict__ mem, const uint2* __restrict__ items,
                                                         uint32_t parity, uint32_t stage, const uint2* __restrict__ epi,
                                                         uint32_t nEpi, uint32_t epiPad)
@@ -49,6 +61,14 @@ __global__ __launch_bounds__(BLK) void k_gradient_batch(const MemberArgs* __rest
     gradientBody<S, MODE, MIX>(M.m, M.p, M.st[parity ^ M.parityFlip][stage], it.y, L.g);
 }
 
+// Cells up to which four lanes take a cell.  The LP limiter's simplex is most of its kernel and its
+// four problems are serial in one lane: always (Euler runs of 1,040 cells 1.87x faster, 10,414 1.73x,
+// 42,496 1.44x, 540,000 1.15x).  The others repeat the cell's weights and ids in every lane, which
+// costs more than the shorter chain gives once the chip is full: FP64 runs of 512 to 32,768 triangles
+// 1.13x to 1.08x, 64,800 1.02x, 99,856 1.01x, 131,072 0.97x, 262,144 0.97x; mixed precision, whose
+// kernel holds more waves, 4,096 1.07x, 19,600 1.03x, 65,536 0.98x.
+static uint32_t quadCells(int mode, int mixed) { return mode == 3 ? ~0u : mixed ? 40000u : 100000u; }
+
 template <int S>
 void gradS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const DiagArgs& d, hipStream_t st)
 {
@@ -56,6 +76,20 @@ void gradS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const Diag
     const uint32_t g = (m.N + BLK - 1) / BLK + pad;
     if (g == 0) return;
     const int mode = p.order == 1 ? 0 : (!(p.limited && a.limit) ? 1 : (p.venkat ? 4 : (p.lpThresh > 0 ? 3 : 2)));
+    if (mode && m.N <= quadCells(mode, p.mixed)) {
+        const dim3 gq((m.N + BLK / 4 - 1) / (BLK / 4) + pad), b(BLK);
+#define EBB_QUAD(MODE, MIX) hipLaunchKernelGGL((k_gradient_quad<S, MODE, MIX>), gq, b, 0, st, m, p, a, d, pad); return
+        switch (mode + 8 * p.mixed) {
+        case 1: EBB_QUAD(1, 0);
+        case 2: EBB_QUAD(2, 0);
+        case 3: EBB_QUAD(3, 0);
+        case 4: EBB_QUAD(4, 0);
+        case 9: EBB_QUAD(1, 1);
+        case 12: EBB_QUAD(4, 1);
+        default: EBB_QUAD(2, 1);
+        }
+#undef EBB_QUAD
+    }
 #define EBB_GRAD(MODE, MIX) hipLaunchKernelGGL((k_gradient<S, MODE, MIX>), dim3(g), dim3(BLK), 0, st, m, p, a, d, pad); break
     if (p.mixed) {
         switch (mode) {
@@ -69,9 +103,8 @@ void gradS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const Diag
     switch (mode) {
     case 0: EBB_GRAD(0, 0);
     case 1: EBB_GRAD(1, 0);
-    case 2: EBB_GRAD(2, 0);
     case 4: EBB_GRAD(4, 0);
-    default: EBB_GRAD(3, 0);
+    default: EBB_GRAD(2, 0);
     }
 #undef EBB_GRAD
 }
