@@ -300,9 +300,11 @@ void launchEpilogue(const DiagArgs& d, hipStream_t stream);
 void launchInitScalars(DevScalars* sc, double dt, double t, double CFL, hipStream_t stream);
 
 // before a residual or step outside the run loop: Rmax starts from rmaxBits, the error words are
-// cleared, and the step's dt is *dt where given; launchEndCall puts the run loop's dt back
+// cleared, and the step's dt is *dt where given.  launchFinishCall: newDt and Rmax from the stages'
+// partials, the run loop's dt put back (putDt), the scalars into the host's page-locked `host`
 void launchBeginCall(DevScalars* sc, unsigned long long rmaxBits, const double* dt, hipStream_t stream);
-void launchEndCall(DevScalars* sc, hipStream_t stream);
+void launchFinishCall(const double* partial, uint32_t nPart, uint32_t nStages, DevScalars* sc, int putDt,
+                      DevScalars* host, hipStream_t stream);
 
 // Batched launches over many meshes (one launch per kernel for all of them).  The kernel
 // shape (S, flux, viscous, order, limiter mode, precision) is the group's; items are

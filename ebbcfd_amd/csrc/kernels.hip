@@ -267,7 +267,43 @@ __global__ void k_begin_call(DevScalars* sc, unsigned long long rmaxBits, double
     }
 }
 
-__global__ void k_end_call(DevScalars* sc) { sc->dt = sc->loopDt; }
+// The end of a call: newDt of its last stage and Rmax of all from their partials (nPart pairs per
+// stage), the run loop's dt put back, and the scalars straight into the host's page-locked copy.  A
+// reduction per stage, a kernel for dt and a copy of the scalars were three to six dependent launches.
+__global__ __launch_bounds__(1024) void k_finish_call(const double* __restrict__ partial, uint32_t nPart, uint32_t nStages,
+                                                      DevScalars* sc, int putDt, DevScalars* host)
+{
+    __shared__ double sMin[16], sMax_[16];
+    __shared__ DevScalars out;
+    double a0 = INFINITY, b0 = 0.0;
+    const uint32_t n = nStages * nPart, lastStage = n - nPart;
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
+        const double2 v = reinterpret_cast<const double2*>(partial)[k];
+        if (k >= lastStage) a0 = fmin(a0, v.x);
+        b0 = fmax(b0, v.y);
+    }
+    a0 = warpMin(a0);
+    b0 = warpMax(b0);
+    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+    if (l == 0) { sMin[w] = a0; sMax_[w] = b0; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t k = 0; k < blockDim.x / 64; k++) { a0 = fmin(a0, sMin[k]); b0 = fmax(b0, sMax_[k]); }
+        DevScalars v = *sc;
+        v.newDtBits = (unsigned long long)__double_as_longlong(a0);
+        if (b0 > __longlong_as_double((long long)v.rmaxBits)) v.rmaxBits = (unsigned long long)__double_as_longlong(b0);
+        if (putDt) v.dt = v.loopDt;
+        sc->newDtBits = v.newDtBits;
+        sc->rmaxBits = v.rmaxBits;
+        sc->dt = v.dt;
+        out = v;
+    }
+    __syncthreads();
+    static_assert(sizeof(DevScalars) % 8 == 0 && sizeof(DevScalars) / 8 <= 1024, "copied as words by one workgroup");
+    if (threadIdx.x < sizeof(DevScalars) / 8)
+        reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
+            reinterpret_cast<const unsigned long long*>(&out)[threadIdx.x];
+}
 
 // ---------------------------------------------------------------- launchers
 static uint32_t nblk(uint64_t n) { return uint32_t((n + BLK - 1) / BLK); }
@@ -353,7 +389,11 @@ void launchBeginCall(DevScalars* sc, unsigned long long rmaxBits, const double* 
     hipLaunchKernelGGL(k_begin_call, dim3(1), dim3(1), 0, st, sc, rmaxBits, dt ? *dt : 0.0, dt ? 1 : 0);
 }
 
-void launchEndCall(DevScalars* sc, hipStream_t st) { hipLaunchKernelGGL(k_end_call, dim3(1), dim3(1), 0, st, sc); }
+void launchFinishCall(const double* partial, uint32_t nPart, uint32_t nStages, DevScalars* sc, int putDt,
+                      DevScalars* host, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_finish_call, dim3(1), dim3(1024), 0, st, partial, nPart, nStages, sc, putDt, host);
+}
 
 void launchInitScalars(DevScalars* sc, double dt, double t, double CFL, hipStream_t st)
 {

@@ -158,9 +158,11 @@ StageArgs loopStageArgs(ebb_solver* s, int kind, double4* qin, const double4* qn
     return a;
 }
 
-// one residual evaluation + stage update
+// one residual evaluation + stage update; inCall: a stage of a residual or step call, whose
+// launchFinishCall reduces the partials (each stage's in its own region, as in the loop)
 void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qout, int limit, int dtUpdate,
-           int first, int last, int checkActive, double4* R, uint32_t stepId, const DiagArgs* epi = nullptr)
+           int first, int last, int checkActive, double4* R, uint32_t stepId, const DiagArgs* epi = nullptr,
+           bool inCall = false)
 {
     const uint32_t stageId = s->stageCounter++;
     StageArgs a;
@@ -169,6 +171,10 @@ void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qo
         s->stageInStep++;
     } else {
         a = baseStageArgs(s, kind, qin, qn, qout, limit, dtUpdate, first, last, stageId, stepId);
+        if (inCall) {
+            a.deferReduce = 1;
+            a.partial = s->d_partial.p + size_t(s->stageInStep++) * 2 * s->nPart;
+        }
     }
     a.R = R;
     s->stageStep.push_back(stepId);
@@ -212,12 +218,12 @@ std::vector<StageDesc> stepSequence(ebb_solver* s)
 
 // Integrator.step: all stages of one step from qcur() into qnext(); epi: the epilogue of the step
 // before, for the first gradient kernel to carry
-void stepStages(ebb_solver* s, int checkActive, uint32_t stepId, const DiagArgs* epi = nullptr)
+void stepStages(ebb_solver* s, int checkActive, uint32_t stepId, const DiagArgs* epi = nullptr, bool inCall = false)
 {
     s->stageInStep = 0;
     const double4* q = s->qcur();
     for (const StageDesc& x : stepSequence(s)) {
-        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, stepId, epi);
+        stage(s, x.kind, x.in, q, x.out, x.limit, x.dtUpdate, x.first, x.last, checkActive, nullptr, stepId, epi, inCall);
         epi = nullptr;
     }
 }
@@ -258,6 +264,12 @@ int readScalars(ebb_solver* s)
     HIPCHK(hipMemcpyAsync(s->h_sc, s->d_sc, sizeof(DevScalars), hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     return EBB_OK;
+}
+
+// the end of a residual or step call: its scalars are in h_sc once the stream is through
+static void finishCall(ebb_solver* s, uint32_t nPart, int putDt)
+{
+    launchFinishCall(s->d_partial.p, nPart, s->stageInStep, s->d_sc, putDt, s->h_sc, s->stream);
 }
 
 // a new window of stages whose errors the next checkErrors reports
@@ -1243,11 +1255,14 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         beginErrorWindow(s);
         launchBeginCall(s->d_sc, bits, nullptr, s->stream);
-        stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, 0);
+        s->stageInStep = 0;
+        stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, 0, nullptr, true);
+        // (the fused path's residual runs the split kernels)
+        finishCall(s, s->useFaceTiles ? s->nPart : (s->N + 255) / 256, 0);
         HIPCHK(hipGetLastError());
         // the kernel leaves R in the reference numbering
         if (R) HIPCHK(copyRows(s, R, s->d_R.p, size_t(s->N) * sizeof(double4), true));
-        { int rc_ = readScalars(s); if (rc_) return rc_; }
+        HIPCHK(hipStreamSynchronize(s->stream));
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);
         std::memcpy(&rm, &s->h_sc->rmaxBits, 8);
@@ -1265,10 +1280,10 @@ int ebb_step(ebb_solver* s, double* dt, double* rmax)
         beginErrorWindow(s);
         // the step runs with the caller's dt; the run loop's own is put back behind it on the device
         launchBeginCall(s->d_sc, 0, dt, s->stream);
-        stepStages(s, 0, uint32_t(s->stepsTotal));
-        launchEndCall(s->d_sc, s->stream);
+        stepStages(s, 0, uint32_t(s->stepsTotal), nullptr, true);
+        finishCall(s, s->nPart, 1);
         HIPCHK(hipGetLastError());
-        { int rc_ = readScalars(s); if (rc_) return rc_; }
+        HIPCHK(hipStreamSynchronize(s->stream));
         s->cur ^= 1;
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);
