@@ -1117,17 +1117,39 @@ struct FaceSrc {
 };
 
 // ---------------------------------------------------------------- residual + update
+// Exchange between lanes of a row of 16 by DPP moves instead of __shfl_xor, whose two LDS permutes per
+// double kept the LDS pipe busy for a third of a last stage's cell phase.  ROW_X1 and ROW_X2 swap with
+// lane ^ 1 and lane ^ 2; the mirrors reach the other quad of an octet and the other octet of the row,
+// whose lanes all hold the same value by then, so they stand for lane ^ 4 and lane ^ 8 of a butterfly.
+// Every lane of the wave must be active.
+enum { ROW_X1 = 0xB1, ROW_X2 = 0x4E, ROW_X4 = 0x141, ROW_X8 = 0x140 };
+template <int CTRL>
+DEV double rowSwap(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+DEV double laneValue(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
 DEV double warpMin(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-    return v;
+    v = fmin(v, rowSwap<ROW_X1>(v));
+    v = fmin(v, rowSwap<ROW_X2>(v));
+    v = fmin(v, rowSwap<ROW_X4>(v));
+    v = fmin(v, rowSwap<ROW_X8>(v));
+    return fmin(fmin(laneValue(v, 0), laneValue(v, 16)), fmin(laneValue(v, 32), laneValue(v, 48)));
 }
 DEV double warpMax(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    return v;
+    v = fmax(v, rowSwap<ROW_X1>(v));
+    v = fmax(v, rowSwap<ROW_X2>(v));
+    v = fmax(v, rowSwap<ROW_X4>(v));
+    v = fmax(v, rowSwap<ROW_X8>(v));
+    return fmax(fmax(laneValue(v, 0), laneValue(v, 16)), fmax(laneValue(v, 32), laneValue(v, 48)));
 }
 
 // solve.d:1092-1117 + the integrator's stage update for interior cell i, from
@@ -1269,9 +1291,13 @@ DEV void rmsBlockLeaf(bool have, const double qNew[4], const double qOld[4], uin
         o[4 + v] = have ? qNew[v] : 0.0;
     }
 #pragma unroll
-    for (int mm = 1; mm < 16; mm <<= 1)
+    for (int q = 0; q < 8; q++) o[q] = o[q] + rowSwap<ROW_X1>(o[q]);
 #pragma unroll
-        for (int q = 0; q < 8; q++) o[q] = o[q] + __shfl_xor(o[q], mm, 64);
+    for (int q = 0; q < 8; q++) o[q] = o[q] + rowSwap<ROW_X2>(o[q]);
+#pragma unroll
+    for (int q = 0; q < 8; q++) o[q] = o[q] + rowSwap<ROW_X4>(o[q]);
+#pragma unroll
+    for (int q = 0; q < 8; q++) o[q] = o[q] + rowSwap<ROW_X8>(o[q]);
     if (have && (threadIdx.x & 15u) == 0) {
         double* dst = rmsBlocks + size_t(refCell / 16) * 8;
         *reinterpret_cast<double4*>(dst) = make_double4(o[0], o[1], o[2], o[3]);
