@@ -135,6 +135,10 @@ struct StageArgs {
     int spec;              // first stage of a time-loop step whose gradient kernel also carries the epilogue
                            // of the step before: that kernel runs as long as the step before ran, and the
                            // tile (or face) kernel after it passes on whether the loop goes on
+    int callBegin;         // first stage of a residual or step call whose gradient kernel does what
+    int callSetDt;         // launchBeginCall would (the error words are clear): Rmax starts from callRmax
+    unsigned long long callRmax;   // and, with callSetDt, the step's dt is callDt
+    double callDt;
     double4* ghostSave;    // spec: receives the ghost rows the gradient kernel replaces, so that a loop that
                            // turns out to have ended gets them back
 };

@@ -697,6 +697,21 @@ DEV bool stageRuns(const StageArgs& a)
     return !a.checkActive || (a.spec ? a.sc->specActive : a.sc->active);
 }
 
+// What one thread of a stage's gradient kernel sets before the stage's other kernels.  Rmax is per step
+// (the time loop's epilogue takes it from the stages' partials instead).  A launch of its own in front
+// of a residual or step call took 5 us.
+DEV void stageBegin(const StageArgs& a)
+{
+    if (a.first && !a.checkActive) a.sc->rmaxBits = 0;
+    if (a.callBegin) {
+        a.sc->rmaxBits = a.callRmax;
+        if (a.callSetDt) {
+            a.sc->loopDt = a.sc->dt;
+            a.sc->dt = a.callDt;
+        }
+    }
+}
+
 // whether the tile or face kernel of a stage runs; one thread of a step's first one passes a loop
 // that has ended on to the next step's gradient kernel
 DEV bool fluxRuns(const StageArgs& a, bool first)
@@ -716,8 +731,7 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     auto& sg = L.sg;
     auto& sl = L.sl;
     if (!stageRuns(a)) return;
-    // Rmax is per step (the time loop's epilogue takes it from the stages' partials instead)
-    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;
+    if (bid == 0 && threadIdx.x == 0) stageBegin(a);
     const uint32_t i = bid * BLK + threadIdx.x;
     if (MODE == 0 && i >= m.N) return;
     const bool have = i < m.N;   // no early return below: the staged stores need every thread
@@ -801,7 +815,7 @@ DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs
 {
     using R = RealOf<MIX>;
     if (!stageRuns(a)) return;
-    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;   // Rmax is per step
+    if (bid == 0 && threadIdx.x == 0) stageBegin(a);
     const uint32_t i = bid * (BLK / 4) + threadIdx.x / 4, v = threadIdx.x & 3u;
     if (i >= m.N) return;
     const R* rows;

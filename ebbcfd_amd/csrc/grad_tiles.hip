@@ -29,7 +29,7 @@ DEV void borderGradBody(const DevMesh& m, const PhysParams& p, const StageArgs& 
 {
     using R = RealOf<MIX>;
     if (!stageRuns(a)) return;
-    if (bid == 0 && threadIdx.x == 0 && a.first && !a.checkActive) a.sc->rmaxBits = 0;   // Rmax is per step
+    if (bid == 0 && threadIdx.x == 0) stageBegin(a);
     const uint32_t k = bid * BLK + threadIdx.x;
     if (k >= t.nBorder) return;
     const uint32_t i = t.border[k];

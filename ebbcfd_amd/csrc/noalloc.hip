@@ -65,6 +65,7 @@ extern "C" int ebb_residual_noalloc(ebb_solver* s, int limit, int dt_update, dou
         unsigned long long bits = 0;
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         // a kernel, not a host copy, so the call needs no synchronisation before its launches
+        s->errClear = false;
         launchBeginCall(s->d_sc, bits, nullptr, s->stream);
         // the split kernels of ebb_residual, with R to the caller's buffer and the partials in scratch
         StageArgs a{};

@@ -165,6 +165,7 @@ void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qo
            bool inCall = false)
 {
     const uint32_t stageId = s->stageCounter++;
+    if (!inCall) s->errClear = false;
     StageArgs a;
     if (checkActive) {
         a = loopStageArgs(s, kind, qin, qn, qout, limit, dtUpdate, first, last, s->stageInStep, stageId, stepId);
@@ -172,6 +173,8 @@ void stage(ebb_solver* s, int kind, double4* qin, const double4* qn, double4* qo
     } else {
         a = baseStageArgs(s, kind, qin, qn, qout, limit, dtUpdate, first, last, stageId, stepId);
         if (inCall) {
+            a.callBegin = s->callBegin; a.callSetDt = s->callSetDt; a.callRmax = s->callRmax; a.callDt = s->callDt;
+            s->callBegin = 0;   // the first stage only
             a.deferReduce = 1;
             a.partial = s->d_partial.p + size_t(s->stageInStep++) * 2 * s->nPart;
         }
@@ -266,10 +269,27 @@ int readScalars(ebb_solver* s)
     return EBB_OK;
 }
 
-// the end of a residual or step call: its scalars are in h_sc once the stream is through
+// The start of a residual or step call: Rmax, the step's dt and clear error words, set by the first
+// stage's gradient kernel where the words are known to be clear (the fused path has no such kernel).
+static void beginCall(ebb_solver* s, unsigned long long rmaxBits, const double* dt)
+{
+    s->stageInStep = 0;
+    s->callBegin = s->errClear && !s->useTiles && s->N > 0;
+    s->callSetDt = dt ? 1 : 0;
+    s->callRmax = rmaxBits;
+    s->callDt = dt ? *dt : 0.0;
+    if (!s->callBegin) launchBeginCall(s->d_sc, rmaxBits, dt, s->stream);
+    s->errClear = false;
+}
+
+// the end of the call: its scalars are in h_sc once the stream is through (callDone)
 static void finishCall(ebb_solver* s, uint32_t nPart, int putDt)
 {
     launchFinishCall(s->d_partial.p, nPart, s->stageInStep, s->d_sc, putDt, s->h_sc, s->stream);
+}
+static void callDone(ebb_solver* s)
+{
+    s->errClear = s->h_sc->errEdge == ~0ull && s->h_sc->errCell == ~0ull && s->h_sc->errBC == ~0ull;
 }
 
 // a new window of stages whose errors the next checkErrors reports
@@ -1254,8 +1274,7 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
         unsigned long long bits = 0;
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         beginErrorWindow(s);
-        launchBeginCall(s->d_sc, bits, nullptr, s->stream);
-        s->stageInStep = 0;
+        beginCall(s, bits, nullptr);
         stage(s, SK_RESIDUAL, s->qcur(), s->qcur(), nullptr, limit, dt_update, 0, 0, 0, s->d_R.p, 0, nullptr, true);
         // (the fused path's residual runs the split kernels)
         finishCall(s, s->useFaceTiles ? s->nPart : (s->N + 255) / 256, 0);
@@ -1263,6 +1282,7 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
         // the kernel leaves R in the reference numbering
         if (R) HIPCHK(copyRows(s, R, s->d_R.p, size_t(s->N) * sizeof(double4), true));
         HIPCHK(hipStreamSynchronize(s->stream));
+        callDone(s);
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);
         std::memcpy(&rm, &s->h_sc->rmaxBits, 8);
@@ -1279,11 +1299,12 @@ int ebb_step(ebb_solver* s, double* dt, double* rmax)
         HIPCHK(hipSetDevice(s->device));
         beginErrorWindow(s);
         // the step runs with the caller's dt; the run loop's own is put back behind it on the device
-        launchBeginCall(s->d_sc, 0, dt, s->stream);
+        beginCall(s, 0, dt);
         stepStages(s, 0, uint32_t(s->stepsTotal), nullptr, true);
         finishCall(s, s->nPart, 1);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s->stream));
+        callDone(s);
         s->cur ^= 1;
         double nd, rm;
         std::memcpy(&nd, &s->h_sc->newDtBits, 8);
@@ -1645,6 +1666,7 @@ int ebb_time_steps(ebb_solver* s, int steps, double out[6])
         if (!s || !out || steps <= 0) return EBB_ERR_ARG;
         HIPCHK(hipSetDevice(s->device));
         { int rc_ = readScalars(s); if (rc_) return rc_; }
+        s->errClear = false;
         DevScalars saved = *s->h_sc;
         const int nst = stagesPerStep(s->cfg);
         std::vector<hipEvent_t> ev(size_t(steps) * nst * 3 + 1);

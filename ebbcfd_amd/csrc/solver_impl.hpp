@@ -149,6 +149,12 @@ struct ebb_solver {
     // stage partials: pairs per stage (the stage kernel's workgroups), region stride,
     // and the stage of the current time-loop step
     uint32_t nPart = 0, pstride = 0, stageInStep = 0;
+    // residual and step calls: no stage has run since a call that left the device's error words clear;
+    // what the next stage's gradient kernel sets for the call (StageArgs::callBegin)
+    bool errClear = false;
+    int callBegin = 0, callSetDt = 0;
+    unsigned long long callRmax = 0;
+    double callDt = 0;
     int64_t stepsTotal = 0;
     double t0 = 0, dt0 = 0;
     std::vector<double> history;     // HIST_FIELDS per completed step of ebb_run

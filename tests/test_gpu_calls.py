@@ -33,3 +33,27 @@ def test_calls_between_runs(integrator, path, nx, ny):
     oh, ot, odt = om.run(3, t=ot, dt=odt)
     assert np.array_equal(h, oh) and (t, dt) == (ot, odt)
     assert np.array_equal(s.q, om.q[:n])
+
+
+@pytest.mark.parametrize("path", ["faceTiles", "split", "fused", "gradTiles"])
+def test_a_failed_call_does_not_reach_the_next(path):
+    from ebbcfd_amd import Solver, build_mesh
+    raw, cfg = channel_case(12, 5, integrator="RK2_TVD")
+    cfg["extensions"] = {"stagePath": path}
+    mesh = build_mesh(raw)
+    s, ref = Solver(mesh, cfg), Solver(mesh, cfg)
+    q = s.q
+    bad = q.copy()
+    bad[7, 0] = -1.0
+    for call in (lambda x: x.step(1e-4), lambda x: x.ufvm_solver()):
+        s.q = q
+        s.step(1e-4)
+        s.q = bad
+        for _ in range(2):
+            with pytest.raises(Exception):
+                call(s)
+        s.q = q
+        ref.q = q
+        for x, y in zip(call(s), call(ref)):
+            assert np.array_equal(x, y)
+        assert np.array_equal(s.q, ref.q)
