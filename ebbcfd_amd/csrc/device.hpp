@@ -722,7 +722,7 @@ DEV bool fluxRuns(const StageArgs& a, bool first)
 }
 
 // One workgroup of the gradient kernel on cell block `bid` of its mesh (the solo and the
-// batched kernels run this same code).  Not MODE 3: the LP limiter runs in gradientQuadBody.
+// batched kernels run this same code).  Not MODE 3: the LP limiter runs in gradientSplitBody.
 template <int S, int MODE, int MIX>
 DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid, GradLds<MODE>& L)
 {
@@ -806,17 +806,20 @@ DEV void gradientBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
     // MODE 1 (unlimited stage): every limiter is 1; the face kernels take LP = 2 and read none
 }
 
-// One workgroup of the gradient kernel with four lanes per cell, one per variable, on block `bid` of
-// BLK / 4 cells: the variables' gradients, bounds and limiters do not depend on each other (a boundary
-// cell's lanes each form the whole ghost state), and a cell's row of four is still one access.  Four
-// times the workgroups with a shorter chain each, for meshes that leave the chip idle.
-template <int S, int MODE, int MIX>
-DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid)
+// One workgroup of the gradient kernel with LANES lanes per cell (4: a variable each, 2: two each) on
+// block `bid` of BLK / LANES cells: the variables' gradients, bounds and limiters do not depend on each
+// other (a boundary cell's lanes each form the whole ghost state), and a cell's row of four is still one
+// access.  More workgroups with a shorter chain and fewer registers each, for meshes that do not fill
+// the chip many times over.
+template <int S, int MODE, int MIX, int LANES>
+DEV void gradientSplitBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, uint32_t bid)
 {
     using R = RealOf<MIX>;
+    constexpr int V = 4 / LANES;
+    typedef R rowV __attribute__((ext_vector_type(V == 1 ? 2 : V)));
     if (!stageRuns(a)) return;
     if (bid == 0 && threadIdx.x == 0) stageBegin(a);
-    const uint32_t i = bid * (BLK / 4) + threadIdx.x / 4, v = threadIdx.x & 3u;
+    const uint32_t i = bid * (BLK / LANES) + threadIdx.x / LANES, v = threadIdx.x % LANES * V;
     if (i >= m.N) return;
     const R* rows;
     if constexpr (MIX == 1) rows = reinterpret_cast<const R*>(a.qin32);
@@ -824,10 +827,20 @@ DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs
     uint32_t nb[S];
 #pragma unroll
     for (int j = 0; j < S; j++) nb[j] = m.nbr[size_t(i) * S + j];
-    R qi[1] = {rows[size_t(i) * 4 + v]}, qn[S][1];
+    auto ldRow = [&](uint32_t c, R o[V]) {
+        if constexpr (V == 2) {
+            const rowV x = *reinterpret_cast<const rowV*>(rows + size_t(c) * 4 + v);
+            o[0] = x[0];
+            o[1] = x[1];
+        } else {
+            o[0] = rows[size_t(c) * 4 + v];
+        }
+    };
+    R qi[V], qn[S][V];
+    ldRow(i, qi);
     double2 cn[S];
 #pragma unroll
-    for (int j = 0; j < S; j++) { qn[j][0] = rows[size_t(nb[j]) * 4 + v]; cn[j] = m.cen[nb[j]]; }
+    for (int j = 0; j < S; j++) { ldRow(nb[j], qn[j]); cn[j] = m.cen[nb[j]]; }
     const double2 ci = m.cen[i];
 #pragma unroll
     for (int j = 0; j < S; j++)
@@ -847,7 +860,12 @@ DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs
                 if (!ok && a.recordErrors) atomicMin(&a.sc->errBC, (uint64_t(a.stageId) << 32) | b);
                 stGhostRow<MIX>(a, nb[j], qg);
             }
-            qn[j][0] = v == 0 ? qg[0] : v == 1 ? qg[1] : v == 2 ? qg[2] : qg[3];
+            if constexpr (V == 2) {
+                qn[j][0] = v ? qg[2] : qg[0];
+                qn[j][1] = v ? qg[3] : qg[1];
+            } else {
+                qn[j][0] = v == 0 ? qg[0] : v == 1 ? qg[1] : v == 2 ? qg[2] : qg[3];
+            }
         }
     bool real[S];
 #pragma unroll
@@ -857,10 +875,18 @@ DEV void gradientQuadBody(const DevMesh& m, const PhysParams& p, const StageArgs
         const double kd = p.venkatK * m.cd[i];
         eps2 = kd * kd * kd;
     }
-    R g[1][2], lx[1], ly[1];
-    gradLimit<S, MODE, R, 1>(qi, qn, nullptr, 0, ci, cn, real, a.limit, p.lpThresh, g, lx, ly, eps2);
+    R g[V][2], lx[V], ly[V];
+    gradLimit<S, MODE, R, V>(qi, qn, nullptr, 0, ci, cn, real, a.limit, p.lpThresh, g, lx, ly, eps2);
     const size_t o = size_t(i) * 4 + v;
-    if constexpr (MIX == 1) {
+    if constexpr (MIX == 1 && V == 2) {
+        __builtin_nontemporal_store((ntf4){g[0][0], g[0][1], g[1][0], g[1][1]}, reinterpret_cast<ntf4*>(a.grad32 + 2 * o));
+        if (MODE == 2 || MODE == 4) *reinterpret_cast<float2*>(a.lim32 + o) = make_float2(lx[0], lx[1]);
+    } else if constexpr (V == 2) {
+        ntd2* gd = reinterpret_cast<ntd2*>(a.grad) + o;
+        __builtin_nontemporal_store((ntd2){g[0][0], g[0][1]}, gd);
+        __builtin_nontemporal_store((ntd2){g[1][0], g[1][1]}, gd + 1);
+        if (MODE == 2 || MODE == 4) __builtin_nontemporal_store((ntd2){lx[0], lx[1]}, reinterpret_cast<ntd2*>(a.lim + o));
+    } else if constexpr (MIX == 1) {
         reinterpret_cast<float2*>(a.grad32)[o] = make_float2(g[0][0], g[0][1]);
         if (MODE == 2 || MODE == 4) a.lim32[o] = lx[0];
     } else {

@@ -31,8 +31,8 @@ __global__ __launch_bounds__(BLK) void k_gradient(DevMesh m, PhysParams p, Stage
     gradientBody<S, MODE, MIX>(m, p, a, (a.order & 2) ? xcdBlockBack(b, nb) : xcdBlock(b, nb), L.g);
 }
 
-template <int S, int MODE, int MIX>
-__global__ __launch_bounds__(BLK) void k_gradient_quad(DevMesh m, PhysParams p, StageArgs a, DiagArgs d, uint32_t epiPad)
+template <int S, int MODE, int MIX, int LANES>
+__global__ __launch_bounds__(BLK) void k_gradient_split(DevMesh m, PhysParams p, StageArgs a, DiagArgs d, uint32_t epiPad)
 {
     __shared__ GradShared<0> L;   // the epilogue's
     if (blockIdx.x < epiPad) {
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(BLK) void k_gradient_quad(DevMesh m, PhysParams p, 
         return;
     }
     const uint32_t b = blockIdx.x - epiPad, nb = gridDim.x - epiPad;
-    gradientQuadBody<S, MODE, MIX>(m, p, a, (a.order & 2) ? xcdBlockBack(b, nb) : xcdBlock(b, nb));
+    gradientSplitBody<S, MODE, MIX, LANES>(m, p, a, (a.order & 2) ? xcdBlockBack(b, nb) : xcdBlock(b, nb));
 }
 
 template <int S, int MODE, int MIX>
@@ -61,13 +61,35 @@ __global__ __launch_bounds__(BLK) void k_gradient_batch(const MemberArgs* __rest
     gradientBody<S, MODE, MIX>(M.m, M.p, M.st[parity ^ M.parityFlip][stage], it.y, L.g);
 }
 
-// Cells up to which four lanes take a cell.  The LP limiter's simplex is most of its kernel and its
-// four problems are serial in one lane: always (Euler runs of 1,040 cells 1.87x faster, 10,414 1.73x,
-// 42,496 1.44x, 540,000 1.15x).  The others repeat the cell's weights and ids in every lane, which
-// costs more than the shorter chain gives once the chip is full: FP64 runs of 512 to 32,768 triangles
-// 1.13x to 1.08x, 64,800 1.02x, 99,856 1.01x, 131,072 0.97x, 262,144 0.97x; mixed precision, whose
-// kernel holds more waves, 4,096 1.07x, 19,600 1.03x, 65,536 0.98x.
-static uint32_t quadCells(int mode, int mixed) { return mode == 3 ? ~0u : mixed ? 40000u : 100000u; }
+// Lanes per cell.  The LP limiter's simplex is most of its kernel and its four problems are serial in
+// one lane: always four (Euler runs of 1,040 cells 1.87x faster, 10,414 1.73x, 42,496 1.44x, 540,000
+// 1.15x).  The other limiters' lanes repeat the cell's ids and weights, which the shorter chain and
+// the smaller register count outweigh until the chip is full several times over.  Runs of one / two /
+// four lanes, us: FP64 8,192 cells 1873 / - / 1687, 32,400: 721 / 706 / 708, 42,496: 1358 / 1281 /
+// 1299, 99,856: 971 / 961 / 1011, 299,266: 3202 / 3037 / - (its limited gradient kernel 16.4 / 13.9),
+// 698,368: 6479 / 6300 / -, 1,048,576: 4551 / 4576 / -; mixed precision 32,400: 675 / 682 / 661,
+// 81,900: 1552 / 1509 / 1553, 698,368: 4639 / 4527 / -, 1,048,576: 3351 / 3401 / -.
+static int gradLanes(int mode, uint32_t cells) { return mode == 3 || cells <= 40000 ? 4 : cells <= 800000 ? 2 : 1; }
+
+template <int S, int LANES>
+static void gradSplit(int mode, const DevMesh& m, const PhysParams& p, const StageArgs& a, const DiagArgs& d,
+                      uint32_t pad, hipStream_t st)
+{
+    const dim3 g((m.N + BLK / LANES - 1) / (BLK / LANES) + pad), b(BLK);
+#define EBB_SPLIT(MODE, MIX) \
+    hipLaunchKernelGGL((k_gradient_split<S, MODE, MIX, LANES>), g, b, 0, st, m, p, a, d, pad); break
+    switch (mode + 8 * p.mixed) {
+    case 1: EBB_SPLIT(1, 0);
+    case 2: EBB_SPLIT(2, 0);
+    case 4: EBB_SPLIT(4, 0);
+    case 9: EBB_SPLIT(1, 1);
+    case 10: EBB_SPLIT(2, 1);
+    case 12: EBB_SPLIT(4, 1);
+    default:
+        if constexpr (LANES == 4) EBB_SPLIT(3, 0);
+    }
+#undef EBB_SPLIT
+}
 
 template <int S>
 void gradS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const DiagArgs& d, hipStream_t st)
@@ -76,20 +98,9 @@ void gradS(const DevMesh& m, const PhysParams& p, const StageArgs& a, const Diag
     const uint32_t g = (m.N + BLK - 1) / BLK + pad;
     if (g == 0) return;
     const int mode = p.order == 1 ? 0 : (!(p.limited && a.limit) ? 1 : (p.venkat ? 4 : (p.lpThresh > 0 ? 3 : 2)));
-    if (mode && m.N <= quadCells(mode, p.mixed)) {
-        const dim3 gq((m.N + BLK / 4 - 1) / (BLK / 4) + pad), b(BLK);
-#define EBB_QUAD(MODE, MIX) hipLaunchKernelGGL((k_gradient_quad<S, MODE, MIX>), gq, b, 0, st, m, p, a, d, pad); return
-        switch (mode + 8 * p.mixed) {
-        case 1: EBB_QUAD(1, 0);
-        case 2: EBB_QUAD(2, 0);
-        case 3: EBB_QUAD(3, 0);
-        case 4: EBB_QUAD(4, 0);
-        case 9: EBB_QUAD(1, 1);
-        case 12: EBB_QUAD(4, 1);
-        default: EBB_QUAD(2, 1);
-        }
-#undef EBB_QUAD
-    }
+    const int lanes = mode ? gradLanes(mode, m.N) : 1;
+    if (lanes == 4) { gradSplit<S, 4>(mode, m, p, a, d, pad, st); return; }
+    if (lanes == 2) { gradSplit<S, 2>(mode, m, p, a, d, pad, st); return; }
 #define EBB_GRAD(MODE, MIX) hipLaunchKernelGGL((k_gradient<S, MODE, MIX>), dim3(g), dim3(BLK), 0, st, m, p, a, d, pad); break
     if (p.mixed) {
         switch (mode) {

@@ -1,5 +1,5 @@
-"""Gradients with four lanes per cell (small meshes) and one lane per cell: the same solve as the
-gradient tiles', which form them in the tile kernel, at the edges of the blocks and of the rule."""
+"""Gradients with four, two and one lane per cell (by the mesh's size): the same solve as the gradient
+tiles', which form them in the tile kernel, at the edges of the blocks and of the rule."""
 import numpy as np
 import pytest
 
@@ -9,12 +9,12 @@ from helpers import channel_case
 pytestmark = pytest.mark.gpu
 
 
-# cells: 1 short block, 64 (a whole block of quads), 65, 256, 257 and, on triangles, both sides of the
-# rule's lines (40,000 and 100,000)
+# cells: 1 short block, 64 (a whole block of four lanes), 65, 256, 257 and, on triangles, both sides of
+# the rule's lines (40,000 and 800,000) and sizes between them
 @pytest.mark.parametrize("limiter", ["scalar", "venkatakrishnan"])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("nx,ny,quads", [(7, 3, 1), (64, 1, 1), (65, 1, 1), (128, 1, 0), (257, 1, 1), (200, 100, 0),
-                                         (201, 100, 0), (500, 100, 0), (501, 100, 0)])
+                                         (201, 100, 0), (500, 100, 0), (501, 100, 0), (1000, 400, 0), (1001, 400, 0)])
 def test_lanes_per_cell_do_not_show(nx, ny, quads, precision, limiter):
     from ebbcfd_amd import Solver, build_mesh
     raw, cfg = channel_case(nx, ny, integrator="RK2_TVD")
