@@ -45,15 +45,32 @@ struct Fold {
     }
 };
 
+template <int CTRL>
+DEV sum2 rowSwap2(sum2 v) { return sum2{rowSwap<CTRL>(v.x), rowSwap<CTRL>(v.y)}; }
+
 // The perfect trees of n items (lane l holds item l, n < 2^levels or all 2^levels), smallest
 // first: for every set bit j of n, the tree over the aligned run of 2^j items that the binary
 // counter keeps at level j.  The xor butterfly adds exactly as the pairwise tree does (the two
-// orders of each sum are equal).
+// orders of each sum are equal); within a row it runs on DPP moves, and a tree's value is read from
+// its lane (n is the same in every lane): LDS permutes took 0.1 us a level in this chain.
 DEV void foldLanes(sum2 x, uint32_t n, int levels, Fold& f)
 {
+    if (n == 0) return;
+    auto take = [&](int j) {
+        const int l = int((n >> (j + 1)) << (j + 1));
+        if (n >> j & 1u) f.add(sum2{laneValue(x.x, l), laneValue(x.y, l)});
+    };
+    take(0);
+    x += rowSwap2<ROW_X1>(x);
+    take(1);
+    x += rowSwap2<ROW_X2>(x);
+    take(2);
+    x += rowSwap2<ROW_X4>(x);
+    take(3);
+    x += rowSwap2<ROW_X8>(x);
 #pragma unroll 1
-    for (int j = 0; j < levels; j++) {
-        if (n >> j & 1u) f.add(shfl2(x, int((n >> (j + 1)) << (j + 1))));
+    for (int j = 4; j < levels && n >> j; j++) {
+        take(j);
         x += shfl2(x, int((threadIdx.x & 63u) ^ (1u << j)));
     }
     if (n >> levels) f.add(x);
@@ -72,8 +89,12 @@ DEV void foldItems(const double* items, uint32_t cnt, Fold& f)
     };
     sum2 y = {0, 0}, g = {0, 0};
     if (lane < tail) y = load(items + size_t(n16) * 128 + lane * 8);
+    if (n16 == 0) {
+        foldLanes(y, tail, 4, f);
+        return;
+    }
     // a lane's sixteen items, eight at a time: the registers of sixteen would cost the gradient
-    // kernel a wave per SIMD in mixed precision
+    // kernel waves in mixed precision (94 registers, set by this code)
 #pragma unroll 1
     for (int h = 0; h < 2; h++) {
         sum2 x[8];
@@ -93,7 +114,17 @@ DEV void foldItems(const double* items, uint32_t cnt, Fold& f)
 // The boundary force sum of mesh.d:645-671: (len*flux) momentum components of the force faces
 // added in order, x in lane 0 and y in lane 1 (their result), so each addition of a chain waits
 // only for its own predecessor.  fp: LDS staging, FORCE_LDS values per component.
-DEV double orderedForce(const uint32_t* faces, uint32_t nF, const double* lenF, double* fp)
+// fi: the first pass's ids, loaded (forceIds) before anything else of the epilogue was waited for.
+constexpr int FS = FORCE_LDS / EPT;
+DEV void forceIds(const uint32_t* faces, uint32_t nF, uint32_t k0, uint32_t fi[FS])
+{
+#pragma unroll
+    for (int u = 0; u < FS; u++) {
+        const uint32_t x = k0 + threadIdx.x + uint32_t(u) * EPT;
+        fi[u] = x < nF ? faces[x] : 0u;
+    }
+}
+DEV double orderedForce(const uint32_t* faces, uint32_t nF, const double* lenF, double* fp, uint32_t fi[FS])
 {
     double f = 0;
     for (uint32_t k0 = 0; k0 < nF; k0 += FORCE_LDS) {
@@ -101,13 +132,7 @@ DEV double orderedForce(const uint32_t* faces, uint32_t nF, const double* lenF, 
         __syncthreads();
         // all of a thread's face ids, then all of their fluxes, are loaded before any is
         // used: two round trips per pass instead of two per face
-        constexpr int FS = FORCE_LDS / EPT;
-        uint32_t fi[FS];
-#pragma unroll
-        for (int u = 0; u < FS; u++) {
-            const uint32_t x = threadIdx.x + uint32_t(u) * EPT;
-            fi[u] = x < cnt ? faces[k0 + x] : 0u;
-        }
+        if (k0) forceIds(faces, nF, k0, fi);
         double2 fv[FS];
 #pragma unroll
         for (int u = 0; u < FS; u++) {
@@ -182,6 +207,20 @@ DEV StepScalars loadScalars(const DevScalars* sc)
             sc->errEdge != ~0ull || sc->errCell != ~0ull || sc->errBC != ~0ull};
 }
 
+// the same in every lane: in scalar registers, not in the vector registers that set the gradient
+// kernel's occupancy
+DEV double uniform(double v) { return laneValue(v, 0); }
+DEV int64_t uniform(int64_t v)
+{
+    return int64_t(uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint64_t(v) >> 32)))) << 32 |
+                   uint32_t(__builtin_amdgcn_readfirstlane(int(v))));
+}
+DEV StepScalars uniform(const StepScalars& s)
+{
+    return {uniform(s.t), uniform(s.dt), uniform(s.CFL), uniform(s.residLast), uniform(s.rms0), uniform(s.steps),
+            uniform(s.incIters), __builtin_amdgcn_readfirstlane(int(s.failed)) != 0};
+}
+
 // The remainder's and the partial chunk's trees (ghost slots hold zeros in both states).
 DEV void foldTail(const DiagArgs& d, Fold& f)
 {
@@ -202,10 +241,9 @@ DEV void foldTail(const DiagArgs& d, Fold& f)
 }
 
 // One workgroup, with the step's newDt, Rmax and force sums at hand and f folded over the
-// remainder and the partial chunk (s0: the scalars, when there are no full chunks): folds the full
-// chunks' tops, writes the history row and the
+// remainder and the partial chunk: folds the full chunks' tops, writes the history row and the
 // loop's scalars and applies the stop conditions.
-DEV void finishStep(const DiagArgs& d, StepScalars s0, EpiLds& L, Fold f, double newDt, double Rmax, double f0, double f1)
+DEV void finishStep(const DiagArgs& d, const StepScalars& s0, EpiLds& L, Fold f, double newDt, double Rmax, double f0, double f1)
 {
     DevScalars* sc = d.sc;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, q0 = tid / 64 * 2;
@@ -224,7 +262,6 @@ DEV void finishStep(const DiagArgs& d, StepScalars s0, EpiLds& L, Fold f, double
         }
         while (idx > 0) { --idx; f.add(sum2{st[idx], st[idx]}); }   // this lane's quantity in its own component
     }
-    if (nfull) s0 = loadScalars(sc);
     if (lane < 2) L.tot[q0 + lane] = 0.0 + (lane ? f.s.y : f.s.x);
     __syncthreads();
     if (tid >= 64) return;
@@ -283,9 +320,11 @@ DEV void finishStep(const DiagArgs& d, StepScalars s0, EpiLds& L, Fold f, double
 DEV void epilogueBody(const DiagArgs& d, uint32_t wg, EpiLds& L, double* staging)
 {
     DevScalars* sc = d.sc;
+    const bool single = d.nEpi == 1;
+    uint32_t fi[FS] = {};
+    if (single || wg == 0) forceIds(d.forceFaces, d.nForce, 0, fi);
     if (!sc->active) return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, q0 = tid / 64 * 2;
-    const bool single = d.nEpi == 1;
     const uint64_t nb = uint64_t(d.L) / 16;
     const uint32_t nfull = uint32_t(nb / RMS_CHUNK_BLOCKS);
     double newDt = 0, rmax = 0;
@@ -293,10 +332,10 @@ DEV void epilogueBody(const DiagArgs& d, uint32_t wg, EpiLds& L, double* staging
     if (single || wg == 1) stageReduce(d, L.red, newDt, rmax);
     if (single || wg == 2) foldTail(d, f);
     else if (wg > 2) foldItems<false>(d.blockSums + size_t(wg - 3) * RMS_CHUNK_BLOCKS * 8, RMS_CHUNK_BLOCKS, f);
-    // (loaded after the folds, whose registers set the gradient kernel's occupancy)
-    const StepScalars s0 = loadScalars(sc);
+    StepScalars s0{};
+    if (single) s0 = loadScalars(sc);
     if (single || wg == 0) {
-        const double s = orderedForce(d.forceFaces, d.nForce, d.lenF, staging);
+        const double s = orderedForce(d.forceFaces, d.nForce, d.lenF, staging, fi);
         if (tid < 2) L.fsum[tid] = s;
         __syncthreads();
     }
@@ -312,6 +351,8 @@ DEV void epilogueBody(const DiagArgs& d, uint32_t wg, EpiLds& L, double* staging
         __syncthreads();
         if (!L.last) return;
         if (tid == 0) sc->ticket = 0;
+        // the scalars and what the others handed over arrive together
+        s0 = loadScalars(sc);
         const double* tail = d.chunkTops + size_t(nfull) * 8 + q0;
         f.s = sum2{agentLoad(tail), agentLoad(tail + 1)};
         f.any = uint64_t(nfull) * RMS_CHUNK_BLOCKS * 16 != d.L;
@@ -320,6 +361,7 @@ DEV void epilogueBody(const DiagArgs& d, uint32_t wg, EpiLds& L, double* staging
         if (tid < 2) L.fsum[tid] = agentLoad(&sc->fsum[tid]);
         __syncthreads();
     }
+    s0 = uniform(s0);
     finishStep(d, s0, L, f, newDt, rmax, L.fsum[0], L.fsum[1]);
 }
 
