@@ -178,10 +178,19 @@ DEV void roeFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Pr
     for (int k = 0; k < 4; k++) out[k] = half * (fL[k] + fR[k]) - half * d[k];
 }
 
+// Least sound speed and density for which rusanovFlux<1> stands, with a flux in range (fluxInRange).
+// Such a flux bounds the pressure p, p bounds the energy E (a nonzero p is at least E's last place)
+// and E the momenta, so that h <= E / rhoMin and G1 / a^2 <= 10 E / aMin^2: 1e216 and 1e218 in FP64,
+// 4e37 and 4e36 in FP32.
+template <typename R>
+struct RusanovRange {
+    static constexpr R aMin = sizeof(R) == 8 ? R(1e-50) : R(1e-5);
+    static constexpr R rhoMin = sizeof(R) == 8 ? R(1e-100) : R(1e-12);
+};
+
 // flux.d:66-141 (Roe-type averages, C1 = C2 = 0: central flux + sMax jump)
 // FAST 1 leaves out what the form with C1 = C2 = 0 multiplies by zero (s1 - sm and s2, with G1,
-// G2, h and the speed): the same bits as long as those factors are finite, that is unless the
-// sound speed vanishes; it then gives NaN as the full form does.
+// G2, h and the speed): the same bits as long as those factors are finite, which RusanovRange says.
 template <int FAST, typename R>
 DEV void rusanovFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1,
                      R out[4], R& sMax)
@@ -213,7 +222,9 @@ DEV void rusanovFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], cons
     convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
     R d[4];
     if constexpr (FAST) {
-        const R z = a > R(sizeof(R) == 8 ? 1e-100 : 1e-12) ? sm : R(NAN);
+        using G = RusanovRange<R>;
+        const bool stands = a > G::aMin && fmin(rhoL, rhoR) > G::rhoMin;
+        const R z = stands ? sm : R(NAN);
         d[0] = z * dRho; d[1] = z * dRhoV0; d[2] = z * dRhoV1; d[3] = z * dRhoE;
     } else {
         const R hL = wL.rho(qL[3] + pL), hR = wR.rho(qR[3] + pR);

@@ -174,7 +174,7 @@ DEV void tileCellPhase(const DevMesh& m, const PhysParams& p, const StageArgs& a
 template <typename R>
 DEV bool fluxInRange(const R F[4])
 {
-    constexpr R big = sizeof(R) == 8 ? R(1e100) : R(1e30);
+    constexpr R big = sizeof(R) == 8 ? R(1e100) : R(1e18);
     return fabs(F[0]) < big && fabs(F[1]) < big && fabs(F[2]) < big && fabs(F[3]) < big;
 }
 
