@@ -50,24 +50,29 @@ template <typename R>
 DEV R dmax(R a, R b) { return a < b ? b : a; }
 
 // Division by one denominator, several times.  FAST 0: IEEE division.  FAST 1: one refined
-// reciprocal per denominator and one Markstein correction per quotient (P. Markstein, IBM J. Res.
-// Dev. 34, 1990): the correctly rounded quotient, so the same bits, for normal denominators and
-// quotients that do not underflow.  A zero, subnormal or infinite denominator or an infinite
-// numerator gives NaN, which the flux carries to its caller (interiorFaceFast), who then takes
-// the IEEE form.  A quotient after the first costs 3 instructions instead of 11.
+// reciprocal per denominator, in FP64, which a quotient is formed from in 3 instructions instead of 11.
+// FP64 quotients take one Markstein correction (P. Markstein, IBM J. Res. Dev. 34, 1990): correctly
+// rounded, so the same bits, for normal denominators and for numerators whose correction does not
+// underflow (1e-290 and more, or zero; below that the last place may differ).  Denominators and sound
+// speeds near the type's lower end are turned away by FastRange.  FP32 quotients are the product with
+// the FP64 reciprocal, rounded: it is within 2^-51 and a quotient of two FP32 numbers is no nearer than
+// 2^-49 to the middle of two others, so they are the same bits for every denominator but zero and
+// infinity (of subnormal quotients those that are such a middle may differ).  Those two, and an
+// infinite FP64 numerator, give NaN, which the flux carries to its caller (faceTileBody: fluxInRange),
+// who then takes the IEEE form (exactFace).  FP32 reciprocals with FP32 corrections, which lose them
+// from numerators of 2e-31 down, took as long: 100 RK2 steps of 1M cells 18.20 and 18.26 ms.
 template <int FAST, typename R>
 struct Div {
-    R b, r;
+    R b;
+    double r;
     DEV Div() {}
-    DEV explicit Div(R d) : b(d), r(R(0))
+    DEV explicit Div(R d) : b(d), r(0)
     {
-        if constexpr (FAST && sizeof(R) == 8) {
-            const R r0 = __builtin_amdgcn_rcp(b);
-            const R r1 = __builtin_fma(__builtin_fma(-b, r0, R(1)), r0, r0);
-            r = __builtin_fma(__builtin_fma(-b, r1, R(1)), r1, r1);
-        } else if constexpr (FAST) {
-            const R r0 = __builtin_amdgcn_rcpf(b);
-            r = __builtin_fmaf(__builtin_fmaf(-b, r0, R(1)), r0, r0);
+        if constexpr (FAST) {
+            const double bd = double(b);
+            const double r0 = __builtin_amdgcn_rcp(bd);
+            const double r1 = __builtin_fma(__builtin_fma(-bd, r0, 1.0), r0, r0);
+            r = __builtin_fma(__builtin_fma(-bd, r1, 1.0), r1, r1);
         }
     }
     DEV R operator()(R a) const
@@ -76,9 +81,7 @@ struct Div {
             const R q = a * r;
             return __builtin_fma(__builtin_fma(-b, q, a), r, q);
         } else if constexpr (FAST) {
-            const R q = a * r;
-            const R q1 = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
-            return __builtin_fmaf(__builtin_fmaf(-b, q1, a), r, q1);
+            return R(double(a) * r);
         } else {
             return a / b;
         }
@@ -86,8 +89,8 @@ struct Div {
 };
 
 // sqrt, with FAST 1 (FP64) by Goldschmidt's iteration from the hardware's reciprocal root without
-// the scaling that subnormal arguments need: the correctly rounded root, the same bits, for normal
-// arguments; NaN for zero and infinity, which takes the flux to its IEEE form like Div's.
+// the scaling that small arguments need: the correctly rounded root, the same bits, from 1e-290 on;
+// NaN for zero and infinity, which takes the flux to its IEEE form like Div's.
 template <int FAST, typename R>
 DEV R root(R x)
 {
@@ -136,6 +139,19 @@ DEV void convective(R p, R u, R v, R rho, R e, R n0, R n1, R out[4])
     out[3] = (u * (p + e)) * n0 + (v * (p + e)) * n1;
 }
 
+// Least sound speed and density for which the FAST fluxes stand, with a flux in range (fluxInRange).
+// In FP64 they keep the denominators, the arguments of the roots and the pressures clear of Div's and
+// root's lower ends.  For the Rusanov flux they also keep finite what it leaves out: a flux in range
+// bounds the pressure p, p bounds the energy E (a nonzero p is at least E's last place) and E the
+// momenta, so that h <= E / rhoMin and G1 / a^2 <= 10 E / aMin^2: 1e216 and 1e218 in FP64, 4e37 and
+// 4e36 in FP32.
+template <typename R>
+struct FastRange {
+    static constexpr R aMin = sizeof(R) == 8 ? R(1e-50) : R(1e-5);
+    static constexpr R rhoMin = sizeof(R) == 8 ? R(1e-100) : R(1e-12);
+    static DEV bool holds(R a, R rhoL, R rhoR) { return a > aMin && fmin(rhoL, rhoR) > rhoMin; }
+};
+
 // flux.d:224-303
 template <int FAST, typename R>
 DEV void roeFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1, R out[4],
@@ -153,7 +169,8 @@ DEV void roeFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Pr
     const R vel0 = (di * uR + uL) * d1, vel1 = (di * vR + vL) * d1;
     const R u = vel0 * n0 + vel1 * n1;
     const R h = (di * hR + hL) * d1;
-    const R a = root<FAST, R>(R(G_ - 1.0) * (h - half * (vel0 * vel0 + vel1 * vel1)));
+    R a = root<FAST, R>(R(G_ - 1.0) * (h - half * (vel0 * vel0 + vel1 * vel1)));
+    if constexpr (FAST && sizeof(R) == 8) a = FastRange<R>::holds(a, rhoL, rhoR) ? a : R(NAN);
     const R dRhoV0 = rvR0 - rvL0, dRhoV1 = rvR1 - rvL1;
     const R dRho = rhoR - rhoL, dRhoE = qR[3] - qL[3];
     const R eps = R(0.01) * a;
@@ -178,19 +195,9 @@ DEV void roeFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Pr
     for (int k = 0; k < 4; k++) out[k] = half * (fL[k] + fR[k]) - half * d[k];
 }
 
-// Least sound speed and density for which rusanovFlux<1> stands, with a flux in range (fluxInRange).
-// Such a flux bounds the pressure p, p bounds the energy E (a nonzero p is at least E's last place)
-// and E the momenta, so that h <= E / rhoMin and G1 / a^2 <= 10 E / aMin^2: 1e216 and 1e218 in FP64,
-// 4e37 and 4e36 in FP32.
-template <typename R>
-struct RusanovRange {
-    static constexpr R aMin = sizeof(R) == 8 ? R(1e-50) : R(1e-5);
-    static constexpr R rhoMin = sizeof(R) == 8 ? R(1e-100) : R(1e-12);
-};
-
 // flux.d:66-141 (Roe-type averages, C1 = C2 = 0: central flux + sMax jump)
 // FAST 1 leaves out what the form with C1 = C2 = 0 multiplies by zero (s1 - sm and s2, with G1,
-// G2, h and the speed): the same bits as long as those factors are finite, which RusanovRange says.
+// G2, h and the speed): the same bits as long as those factors are finite, which FastRange says.
 template <int FAST, typename R>
 DEV void rusanovFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], const Prim<FAST, R>& wR, R n0, R n1,
                      R out[4], R& sMax)
@@ -222,9 +229,7 @@ DEV void rusanovFlux(const R qL[4], const Prim<FAST, R>& wL, const R qR[4], cons
     convective<R>(pR, uR, vR, rhoR, qR[3], n0, n1, fR);
     R d[4];
     if constexpr (FAST) {
-        using G = RusanovRange<R>;
-        const bool stands = a > G::aMin && fmin(rhoL, rhoR) > G::rhoMin;
-        const R z = stands ? sm : R(NAN);
+        const R z = FastRange<R>::holds(a, rhoL, rhoR) ? sm : R(NAN);
         d[0] = z * dRho; d[1] = z * dRhoV0; d[2] = z * dRhoV1; d[3] = z * dRhoE;
     } else {
         const R hL = wL.rho(qL[3] + pL), hR = wR.rho(qR[3] + pR);

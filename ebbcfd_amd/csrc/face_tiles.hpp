@@ -166,9 +166,9 @@ DEV void tileCellPhase(const DevMesh& m, const PhysParams& p, const StageArgs& a
     blockPartial(dtCand, rCand, a.partial, pslot);
 }
 
-// Whether a face's flux by the FAST forms stands: every quotient outside their range (a zero,
-// subnormal or infinite denominator, a vanishing sound speed) has reached it as a NaN or as a
-// value beyond any flow's.  The forms with a guard on every quotient took longer than plain
+// Whether a face's flux by the FAST forms stands: what is outside their range (a zero or infinite
+// denominator, a density or sound speed below FastRange's) has reached it as a NaN or as a value
+// beyond any flow's.  The forms with a guard on every quotient took longer than plain
 // divisions; this one test takes the 4.2M-cell viscous Rusanov launches from 295 to 265-278 us
 // (VALU issue was ~155 us of them) and a 299,266-cell Roe launch from 33.6 to 32.4 us.
 template <typename R>
