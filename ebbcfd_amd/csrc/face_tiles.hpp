@@ -13,6 +13,7 @@ namespace ebb {
 // of the mesh set-up (source/mesh.d; mesh.cpp), so they equal the stored ones bit
 // for bit.  Interior edges: normal = (y1-y0, x0-x1)/|.|, whose norm is the length
 // (the same squares summed in the other order); boundary edges: (1/len) * (...).
+// FAST: by Div's and root's short forms, for meshes without exactEdges.
 template <int FAST = 0>
 DEV void edgeGeometry(bool interior, double2 p0, double2 p1, double2& n, double2& mid, double& len)
 {
@@ -182,12 +183,11 @@ DEV bool fluxInRange(const R F[4])
 // keep them for it (the opaque record stops the compiler from doing so).
 template <int FLUX, int VISC, int ORDER, int LP, int MIX>
 DEV void exactFace(const DevMesh& m, const PhysParams& p, const FaceSrc<MIX>& src, uint4 r,
-                   typename FaceSrc<MIX>::R F[4], typename FaceSrc<MIX>::R& sMax)
+                   typename FaceSrc<MIX>::R F[4], typename FaceSrc<MIX>::R& sMax, double& len)
 {
     using R = typename FaceSrc<MIX>::R;
     asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z), "+v"(r.w));
     double2 n, mid, ca = make_double2(0, 0), cb = make_double2(0, 0);
-    double len;
     edgeGeometry(true, m.node[r.z], m.node[r.w], n, mid, len);
     R qa[4], qb[4], ga[8], gb[8], lxa[4], lya[4], lxb[4], lyb[4], qL[4], qR[4];
     src.q(r.x, qa);
@@ -253,9 +253,10 @@ DEV void faceTileBody(const DevMesh& m, const PhysParams& p, const StageArgs& a,
         if (interior) {
             interiorFace<FLUX, VISC, ORDER, LP, R, 1>(qa, ga, lxa, lya, ca, qb, gb, lxb, lyb, cb, n, mid, p, qL, qR,
                                                      Fr, sMr);
-            if (!fluxInRange(Fr)) exactFace<FLUX, VISC, ORDER, LP, MIX>(m, p, src, r, Fr, sMr);
+            if (m.exactEdges || !fluxInRange(Fr)) exactFace<FLUX, VISC, ORDER, LP, MIX>(m, p, src, r, Fr, sMr, len);
         } else {
             isB = true;
+            if (m.exactEdges) edgeGeometry(false, m.node[r.z], m.node[r.w], n, mid, len);
             b = r.y - m.N;   // the ghost of boundary face b is cell N + b
             boundaryFace<FLUX, VISC, ORDER, LP, R>(qa, ga, lxa, lya, ca, qb, m.bface[b], n, mid, p, qL, qR, Fr, sMr);
         }
