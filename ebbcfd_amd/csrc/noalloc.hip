@@ -66,6 +66,7 @@ extern "C" int ebb_residual_noalloc(ebb_solver* s, int limit, int dt_update, dou
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         // a kernel, not a host copy, so the call needs no synchronisation before its launches
         s->errClear = false;
+        s->replayable = true;
         launchBeginCall(s->d_sc, bits, nullptr, s->stream);
         // the split kernels of ebb_residual, with R to the caller's buffer and the partials in scratch
         StageArgs a{};

@@ -274,7 +274,7 @@ int readScalars(ebb_solver* s)
 static void beginCall(ebb_solver* s, unsigned long long rmaxBits, const double* dt)
 {
     s->stageInStep = 0;
-    s->callBegin = s->errClear && !s->useTiles && s->N > 0;
+    s->callBegin = s->errClear && !s->replayable && !s->useTiles && s->N > 0;
     s->callSetDt = dt ? 1 : 0;
     s->callRmax = rmaxBits;
     s->callDt = dt ? *dt : 0.0;

@@ -152,6 +152,9 @@ struct ebb_solver {
     // residual and step calls: no stage has run since a call that left the device's error words clear;
     // what the next stage's gradient kernel sets for the call (StageArgs::callBegin)
     bool errClear = false;
+    // an ebb_residual_noalloc was called, which may have been captured: its replays leave error words that
+    // the host knows nothing of, so errClear is not relied on any more
+    bool replayable = false;
     int callBegin = 0, callSetDt = 0;
     unsigned long long callRmax = 0;
     double callDt = 0;
