@@ -1139,11 +1139,17 @@ int ebb_solver_create(const ebb_mesh* m, const ebb_config* c, int device, ebb_so
 }
 
 // A renumbered solver's rows cross the host boundary in the reference numbering: they are
-// permuted on the device, through the residual's buffer.  (Host loops over a permuted copy took
-// 30 ms for the states of 4.2M cells, the kernel takes 0.1 ms.)
-static int rowStaging(ebb_solver* s)
+// permuted on the device, through the face fluxes' buffer, which holds nothing between calls (a stage
+// forms the rows that it reads, and ebb_edge_states those that it returns) and has a row of four per
+// face.  A mesh whose cells share a face by two at most has 1.5 times as many faces as cells; another,
+// with fewer, takes the residual's buffer.  The padding row past the faces stays zero.  (Host loops over a
+// permuted copy took 30 ms for the states of 4.2M cells, the kernel takes 0.1 ms.)
+static int rowStaging(ebb_solver* s, double4** rows)
 {
+    *rows = reinterpret_cast<double4*>(s->d_lenF.p);
+    if (s->Fi + s->Fb >= s->N) return EBB_OK;
     if (!s->d_R.p) HIPCHK((hipError_t)trackAlloc(s, s->d_R, s->N));
+    *rows = s->d_R.p;
     return EBB_OK;
 }
 
@@ -1151,10 +1157,7 @@ static int rowStaging(ebb_solver* s)
 static int uploadStates(ebb_solver* s, const double* host, double4* dev)
 {
     double4* dst = dev;
-    if (!s->refOf.empty()) {
-        { int rc_ = rowStaging(s); if (rc_) return rc_; }
-        dst = s->d_R.p;
-    }
+    if (!s->refOf.empty()) { int rc_ = rowStaging(s, &dst); if (rc_) return rc_; }
     HIPCHK(copyRows(s, const_cast<double*>(host), dst, size_t(s->N) * sizeof(double4), false));
     if (dst != dev) launchPermuteRows(dst, dev, s->d_refId.p, s->N, s->stream);
     HIPCHK(hipGetLastError());
@@ -1167,10 +1170,11 @@ static int downloadStates(ebb_solver* s, const double4* dev, double* host)
 {
     const double4* src = dev;
     if (!s->refOf.empty()) {
-        { int rc_ = rowStaging(s); if (rc_) return rc_; }
-        launchPermuteRows(dev, s->d_R.p, s->d_devOf.p, s->N, s->stream);
+        double4* rows;
+        { int rc_ = rowStaging(s, &rows); if (rc_) return rc_; }
+        launchPermuteRows(dev, rows, s->d_devOf.p, s->N, s->stream);
         HIPCHK(hipGetLastError());
-        src = s->d_R.p;
+        src = rows;
     }
     HIPCHK(copyRows(s, host, const_cast<double4*>(src), size_t(s->N) * sizeof(double4), true));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1274,7 +1278,7 @@ int ebb_residual(ebb_solver* s, int limit, int dt_update, double* R, double* new
     return guarded([&]() -> int {
         if (!s) return EBB_ERR_ARG;
         HIPCHK(hipSetDevice(s->device));
-        { int rc_ = rowStaging(s); if (rc_) return rc_; }
+        if (!s->d_R.p) HIPCHK((hipError_t)trackAlloc(s, s->d_R, s->N));
         unsigned long long bits = 0;
         if (rmax && *rmax > 0) std::memcpy(&bits, rmax, 8);
         beginErrorWindow(s);
@@ -1474,7 +1478,8 @@ int ebb_edge_states(ebb_solver* s, double* eq, double* flux, double* smax)
         std::vector<double4> es(size_t(F) * 2);
         std::vector<double> lf(size_t(F) * 4), ls(F);
         HIPCHK(hipMemcpy(es.data(), s->d_estate.p, es.size() * sizeof(double4), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(lf.data(), s->d_lenF.p, lf.size() * sizeof(double), hipMemcpyDeviceToHost));
+        if (s->haveStage)   // (else no flux yet: zeros)
+            HIPCHK(hipMemcpy(lf.data(), s->d_lenF.p, lf.size() * sizeof(double), hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(ls.data(), s->d_lenS.p, ls.size() * sizeof(double), hipMemcpyDeviceToHost));
         for (uint32_t f = 0; f < F; f++) {
             const uint32_t e = s->edgeOfFace[f];
