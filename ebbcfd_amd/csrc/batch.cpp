@@ -440,6 +440,7 @@ int ebb_batch_add(ebb_batch* b, const ebb_mesh* m, const ebb_config* c, int64_t*
         cfg.stagePath = cfg.stagePath == 3 ? 3 : 1;
         cfg.tileOrder = 2;
         cfg.renumber = false;
+        cfg.batchMember = true;
         // automatic tiles are sized for the cells of the running members and this one
         // together: a member admitted alone or beside small ones spreads over the GPU as a
         // solo run does; one joining members that already fill it takes full-size tiles

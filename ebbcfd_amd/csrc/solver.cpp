@@ -153,7 +153,7 @@ StageArgs loopStageArgs(ebb_solver* s, int kind, double4* qin, const double4* qn
     a.partial = s->d_partial.p + size_t(stageInStep) * 2 * s->nPart;
     if (first && s->rideEpilogue) {
         a.spec = 1;
-        a.ghostSave = s->d_ghostSave.p;   // null on gradient tiles, whose tile kernel stores the ghosts
+        a.ghostSave = s->d_ghostSave.p;   // null on gradient tiles, whose tile kernel stores the ghosts, and in batches
     }
     return a;
 }
@@ -603,7 +603,8 @@ int64_t estimateDeviceBytes(const BuiltMesh& b, const Config& c)
                                             c.spreadTiles ? std::min<int64_t>(N / 32 + 1, 1024) : 0);
     bytes += (2 * std::max<int64_t>((N + 255) / 256, tiles) + 2) * 4 * 8;   // stage partials
     bytes += 256 * HIST_FIELDS * 8;
-    bytes += (C / 16 / RMS_CHUNK_BLOCKS + 1) * 64 + G * 32;   // chunk tops; ghost rows kept for a loop that ends
+    bytes += (C / 16 / RMS_CHUNK_BLOCKS + 1) * 64;         // chunk tops
+    if (!c.batchMember) bytes += G * 32;                   // ghost rows kept for a loop that ends
     return bytes;
 }
 
@@ -785,7 +786,8 @@ int buildDevice(ebb_solver* s)
         for (const BFace& bf : s->bfaces) tpin = tpin || bf.type == TempPresInflow;
         s->rideEpilogue = s->rmsFused && !tpin;
     }
-    if (s->rideEpilogue && !s->useGradTiles) HIPCHK((hipError_t)trackAlloc(s, s->d_ghostSave, s->G));
+    // a batched solve's ghost rows are never read, so an ended one need not get them back
+    if (s->rideEpilogue && !s->useGradTiles && !c.batchMember) HIPCHK((hipError_t)trackAlloc(s, s->d_ghostSave, s->G));
     HIPCHK(hipMalloc((void**)&s->d_sc, sizeof(DevScalars)));
     HIPCHK(hipHostMalloc((void**)&s->h_sc, sizeof(DevScalars), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void**)&s->h_hist, sizeof(double) * size_t(s->histCap) * HIST_FIELDS, hipHostMallocDefault));
