@@ -69,7 +69,6 @@ struct DevMesh {
     const double4* __restrict__ src;     // N MMS source (null if none)
     const uint32_t* __restrict__ refId;  // N: reference index of each device cell
     const double2* __restrict__ node;    // mesh node coordinates
-    uint32_t exactEdges;      // 1: some edge's squared length leaves the range of the face tiles' short forms
 };
 
 struct PhysParams {

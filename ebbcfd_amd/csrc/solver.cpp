@@ -799,10 +799,6 @@ int buildDevice(ebb_solver* s)
     dm.fcell = s->d_fcell.p; dm.fn = s->d_fn.p; dm.fmid = s->d_fmid.p; dm.flen = s->d_flen.p;
     dm.bface = s->d_bface.p; dm.src = c.mms ? s->d_src.p : nullptr; dm.refId = s->d_refId.p;
     dm.node = s->d_node.p;
-    // an edge outside this range has a squared length near the ends of FP64, where root<1> loses its last
-    // place.  Decided once per mesh: a test per face took a 130,143-quadrilateral run from 2.99 to 3.05 ms
-    for (double len : b.len)
-        if (!(len > 1e-100 && len < 1e100)) dm.exactEdges = 1;
 
     // initial state (solve.d:194-207; app/ms.d:295-298)
     std::vector<double4> q0(C, make_double4(0, 0, 0, 0));
