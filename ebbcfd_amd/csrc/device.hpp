@@ -60,7 +60,7 @@ DEV R dmax(R a, R b) { return a < b ? b : a; }
 // infinity (of subnormal quotients those that are such a middle may differ).  Those two, and an
 // infinite FP64 numerator, give NaN, which the flux carries to its caller (faceTileBody: fluxInRange),
 // who then takes the IEEE form (exactFace).  FP32 reciprocals with FP32 corrections, which lose them
-// from numerators of 2e-31 down, took as long: 100 RK2 steps of 1M cells 18.20 and 18.26 ms.
+// from numerators of 2e-31 down, took as long: 100 RK2 steps of 1M cells 18.13 and 18.18 ms.
 template <int FAST, typename R>
 struct Div {
     R b;
@@ -405,7 +405,8 @@ DEV bool ghostState(const BFace& b, const R qo[4], R qg[4], const R qgOld[4])
 // most one row of a pair and each pair costs one product sum and one quotient ((-a)p + (-b)q is
 // -(ap + bq) exactly).  The first row of the smallest ratio is kept while the pairs go by, with
 // its coefficients, instead of being looked up in arrays of rows, ratios and candidates (which
-// lived in scratch memory).  The gradient launch of 10,414 triangles: 88 -> 29 us.
+// lived in scratch memory).  The gradient launch of 10,414 triangles: 88 -> 29 us, and 10 with a lane
+// per variable (gradientSplitBody).
 template <int S>
 DEV void lpSolve(const double ex[S], const double ey[S], const bool real[S], double lo, double hi, double c0, double c1,
                  double& x, double& y)

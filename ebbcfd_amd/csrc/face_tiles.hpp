@@ -173,8 +173,9 @@ DEV void tileCellPhase(const DevMesh& m, const PhysParams& p, const StageArgs& a
 // Whether a face's flux by the FAST forms stands: what is outside their range (a zero or infinite
 // denominator, a density or sound speed below FastRange's) has reached it as a NaN or as a value
 // beyond any flow's.  The forms with a guard on every quotient took longer than plain
-// divisions; this one test takes the 4.2M-cell viscous Rusanov launches from 295 to 265-278 us
-// (VALU issue was ~155 us of them) and a 299,266-cell Roe launch from 33.6 to 32.4 us.
+// divisions; this one test took the 4.2M-cell viscous Rusanov launches from 295 to 265-278 us
+// (VALU issue was ~155 us of them; they take 245 and 265 now, with 108 and 122 us of issue) and a
+// 299,266-cell Roe launch from 33.6 to 32.4 us (26.5 now).
 template <typename R>
 DEV bool fluxInRange(const R F[4])
 {

@@ -10,7 +10,7 @@ namespace ebb {
 // A stage in two launches that keeps most gradient and limiter rows on chip.
 //   k_border_grad  per ring cell (a cell across a face of some other tile): its gradient
 //                  and limiter rows to HBM; it also carries the gradient kernel's other
-//                  duties (the previous step's boundary force, the per-step Rmax reset);
+//                  duties (the epilogue of the step before, a call's first scalars);
 //   k_grad_tile    per tile: its own cells' ghosts, gradients and limiters into LDS, the
 //                  ring cells' rows copied in from the border kernel's output, then every
 //                  face of the tile and the cells' update as in k_face_tile.
@@ -23,7 +23,7 @@ namespace ebb {
 constexpr int GROW = 12;
 
 // One workgroup of the border kernel on border block `bid` of its mesh (the solo and the
-// batched kernels run this same code); block 0 also resets the step's Rmax.
+// batched kernels run this same code); block 0 also sets what a call starts with (stageBegin).
 template <int S, int MODE, int MIX>
 DEV void borderGradBody(const DevMesh& m, const PhysParams& p, const StageArgs& a, const FaceTileArgs& t, uint32_t bid)
 {

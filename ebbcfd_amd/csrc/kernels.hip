@@ -1,6 +1,6 @@
 // HIP kernels for the explicit residual-and-update loop, FP64, gfx950.
 //
-// One residual evaluation (source/solve.d:322-1122) is three launches:
+// One residual evaluation (source/solve.d:322-1122) on the split path is three launches:
 //   k_gradient  per interior cell: ghost states of its boundary faces
 //               (solve.d:520-689), LSQ gradient, min/max bounds and the scalar
 //               limiter at neighbour centroids (solve.d:324-403), LP vector
@@ -11,10 +11,12 @@
 //               (solve.d:769-968); stores len*flux and len*sMax per face;
 //   k_update    per interior cell: gathers its faces in the cell's own edge
 //               order with the owner sign (solve.d:1082-1118), CFL time step
-//               and Rmax (block reduction + one ordered-bits atomic per block,
-//               exact because min/max are order independent), the MMS source
-//               (app/ms.d:131-141) and the integrator stage update
-//               (source/integrators.d:22-270) fused in.
+//               and Rmax (one pair of partials per block, reduced by the step's
+//               epilogue or the call's last kernel; exact because min/max are order
+//               independent), the MMS source (app/ms.d:131-141) and the integrator
+//               stage update (source/integrators.d:22-270) fused in.
+// The default path is two: k_gradient and k_face_tile, which does the work of the other two
+// for a tile of cells with the faces in LDS.
 // No atomics touch the residual: each cell sums its own faces in a fixed order,
 // so results are deterministic and bit-identical to the edge-loop form.
 // Built with -ffp-contract=off: every product and sum rounds as written.

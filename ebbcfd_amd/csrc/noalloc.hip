@@ -68,7 +68,7 @@ extern "C" int ebb_residual_noalloc(ebb_solver* s, int limit, int dt_update, dou
         s->errClear = false;
         s->replayable = true;
         launchBeginCall(s->d_sc, bits, nullptr, s->stream);
-        // the split kernels of ebb_residual, with R to the caller's buffer and the partials in scratch
+        // the split path's kernels, a fixed pair of partials per 256 cells, with R to the caller's buffer
         StageArgs a{};
         a.qin = s->qcur(); a.qn = s->qcur(); a.qout = nullptr; a.acc = s->d_acc.p;
         a.R = reinterpret_cast<double4*>(R_dev);

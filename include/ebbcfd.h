@@ -221,9 +221,10 @@ int ebb_limiter1d(int device, int kind, int64_t n, const double* sp, const doubl
  * the first mesh (source/integrators.d:56-75), so one process holds one mesh.  A batch
  * holds many solvers (each the result of ufvmSetup on its own mesh and config, state
  * resident on the device) and advances all of them with one launch per kernel: per RK
- * stage one gradient launch and one face/update launch over every mesh's blocks and tiles,
- * then one RMS launch and one epilogue launch, the whole step sequence captured as a HIP
- * graph.  Each mesh's states and history equal its solo ebb_run's bit for bit.  Members
+ * stage one gradient launch and one face/update launch over every mesh's blocks and tiles
+ * (the first of a step also carries the epilogues of the step before, unless a member has a
+ * total-conditions inflow: they are a launch of their own then, as after the last step of a
+ * sequence), the whole step sequence captured as a HIP graph.  Each mesh's states and history equal its solo ebb_run's bit for bit.  Members
  * use the face-tile stage path (or the gradient tiles, extensions.stagePath = "gradTiles")
  * in the reference cell numbering; the LP vector limiter and the fused stage path are not
  * batched. */
